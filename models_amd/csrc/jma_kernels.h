@@ -303,12 +303,13 @@ struct QMatArgs {
 // group_rows).
 hipError_t launch_qmatvec(const QMatArgs& a, uint32_t fmt, uint32_t tiles, hipStream_t stream);
 // Prefill-sized batches of the 32-element block formats (fmt 0, 1, 5): the activations quantized
-// once to q (int8 [batch][cols]) and scales ([batch][cols / 32]), then the register-tiled
-// product; tiles = sum of ceil(rows / kQGemmTile), grid tiles x ceil(batch / kQGemmTile).
-hipError_t launch_q8_0_quant(const float* x, uint32_t batch, uint32_t cols, int8_t* q,
-                             float* scales, hipStream_t stream);
-hipError_t launch_qgemm(const QMatArgs& a, uint32_t fmt, uint32_t tiles, const int8_t* aq,
-                        const float* as, hipStream_t stream);
+// once to act (halves, qact_index) and their f16 scales (qact_scale_index), every row up to a
+// multiple of 32 written; then the matrix product in workgroup tiles of kQGemmShape[shape],
+// tiles_w = sum of ceil(rows / qgemm_rows_w).
+hipError_t launch_q8_0_quant(const float* x, uint32_t batch, uint32_t cols, void* act, void* scales,
+                             hipStream_t stream);
+hipError_t launch_qgemm(const QMatArgs& a, uint32_t fmt, uint32_t shape, uint32_t tiles_w,
+                        const void* act, const void* act_scale, hipStream_t stream);
 // The same for Q4_K (fmt 2), Q6_K (fmt 3) and Q5_K (fmt 4) on Q8_K activations: q int8
 // [batch][cols], scales [batch][cols / 256], sums int [batch][cols / 16] (Q6_K reads no sums).
 hipError_t launch_q8_k_quant(const float* x, uint32_t batch, uint32_t cols, int8_t* q,

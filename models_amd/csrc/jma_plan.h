@@ -274,12 +274,80 @@ constexpr uint64_t kQMatLds = 64u * 1024u;   // dynamic LDS a projection workgro
 constexpr uint32_t kQMatMaxChunk = 8;        // activation rows per pass
 constexpr uint32_t kQMatTargetBlocks = 1024;  // workgroups a projection launch aims for
 
-// Batches of at least kQGemmMinBatch activation rows run as a register-tiled product
-// (qgemm_kernel, qkgemm_kernel, q6gemm_kernel): tiles of kQGemmTile weight rows x kQGemmTile
-// activation rows, kQGemmKc 32-element blocks (or one 256-element block) staged per step.
+// Batches of at least kQGemmMinBatch activation rows run as a matrix product on the matrix cores
+// (jma_qgemm.hip) over activations quantized once into scratch.
 constexpr uint32_t kQGemmMinBatch = 16;
-constexpr uint32_t kQGemmTile = 64;
-constexpr uint32_t kQGemmKc = 4;
+
+// Quantized activations of a product, as halves (the int8 values exactly) in the order the matrix
+// ops read them: tiles of 32 activation rows; per tile, chunks of 16 inputs, each [k half h][row]
+// [8 inputs], so the 64 lanes (32 h + row) of one operand load read 1 KB in order. Element index
+// of input k of row b:
+JMA_HD uint64_t qact_index(uint32_t b, uint32_t k, uint32_t cols) {
+  return (uint64_t)(b / 32u) * 32u * cols + (uint64_t)(k / 16u) * 512u + ((k / 8u) % 2u) * 256u +
+         (b % 32u) * 8u + k % 8u;
+}
+// Scale of block blk (of K per row) of row b.
+JMA_HD uint64_t qact_scale_index(uint32_t b, uint32_t blk, uint32_t K) {
+  return (uint64_t)(b / 32u) * 32u * K + (uint64_t)blk * 32u + b % 32u;
+}
+JMA_HD uint32_t qact_tiles(uint32_t batch) { return (batch + 31u) / 32u; }
+
+// Bytes of the activations of a batch (32-row tiles), rounded up to keep what follows aligned.
+JMA_HD uint64_t qact_bytes(uint32_t batch, uint32_t cols) {
+  return ((uint64_t)qact_tiles(batch) * 32u * cols * 2u + 255u) / 256u * 256u;
+}
+// Scratch to hold for calls of up to `elements` = batch x cols activations, whatever their format
+// and shape, so that a captured call no larger than an eager one before it never has to grow it:
+// rounding a batch of 16 or more up to 32 rows at most doubles it; scales and sums take at most
+// 1/4 + 1/32 of a byte per byte of int8 (Q8_K: one f32 per 256, one 16-bit sum per 16).
+JMA_HD uint64_t qact_reserve_bytes(uint64_t elements) { return elements * 4u + elements / 2u + 4096u; }
+
+// Workgroup tiles of the product: 32 bt nb activation rows x 32 wt nw weight rows on nb x nw
+// waves of bt x wt 32 x 32 tiles each, half a weight block staged per thread and step.
+struct QGemmShape {
+  uint32_t bt, wt, nb, nw;
+};
+constexpr uint32_t qgemm_rows_b(QGemmShape s) { return 32u * s.bt * s.nb; }
+constexpr uint32_t qgemm_rows_w(QGemmShape s) { return 32u * s.wt * s.nw; }
+constexpr uint32_t qgemm_threads(QGemmShape s) { return 64u * s.nb * s.nw; }
+constexpr uint32_t kQGemmTile = 64;  // K-quants
+constexpr uint32_t kQGemmShapes = 3;
+constexpr QGemmShape kQGemmShape[kQGemmShapes] = {
+    {2, 2, 2, 2},  // 128 x 128
+    {1, 1, 2, 2},  // 64 x 64
+    {1, 1, 1, 4},  // 32 x 128
+};
+
+// Tile (tx, ty) of workgroup `id` of a launch of `total` = tiles_w x batch tiles: the workgroups
+// of one XCD (dispatch order modulo 8) take consecutive tiles, the weight tiles fastest, so that
+// an XCD's L2 keeps the activations of few batch tiles. recip = qgemm_recip(tiles_w): the quotient
+// by it is exact or one short, and stays on the scalar unit (a division goes through the vector
+// unit's reciprocal, and the buffer descriptors made from it would be built in vector registers).
+inline uint32_t qgemm_recip(uint32_t tiles_w) {
+  return tiles_w <= 1 ? 0xFFFFFFFFu : (uint32_t)(((uint64_t)1 << 32) / tiles_w);
+}
+JMA_HD void qgemm_tile(uint32_t id, uint32_t tiles_w, uint32_t recip, uint32_t total, uint32_t& tx,
+                       uint32_t& ty) {
+  const uint32_t xcd = id % 8u, per = total / 8u, rem = total % 8u;
+  const uint32_t t = xcd * per + (xcd < rem ? xcd : rem) + id / 8u;
+  ty = (uint32_t)(((uint64_t)t * recip) >> 32);
+  tx = t - ty * tiles_w;
+  if (tx >= tiles_w) {
+    tx -= tiles_w;
+    ++ty;
+  }
+}
+
+// The workgroup tile (index of kQGemmShape) of a product launch: the largest once its tiles cover
+// half the compute units (1000 rows: 3072 outputs of 3072 inputs, 192 tiles, 68 us against 73 with
+// 64 x 64 tiles; 512 rows, 96 tiles, 46 against 39), else the small ones, 32 rows wide for batches
+// that fit.
+inline uint32_t plan_qgemm(const uint32_t* rows, uint32_t count, uint32_t batch, uint32_t cus) {
+  uint64_t tiles = 0;
+  for (uint32_t i = 0; i < count; ++i) tiles += (rows[i] + 127u) / 128u;
+  if (tiles * ((batch + 127u) / 128u) * 2 >= cus) return 0;
+  return batch <= 32 ? 2 : 1;
+}
 
 struct QMatPlan {
   uint32_t rows_per_tile = 0, chunk = 0;  // 0: cols too large for one workgroup's LDS

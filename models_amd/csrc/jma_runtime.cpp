@@ -827,25 +827,22 @@ void quantized_matmul_impl(jmodels_attn_context* ctx, const std::vector<QuantMat
               std::to_string((uint64_t)batch * total_rows));
   // Launches, one per weight format of the call. Prefill-sized batches quantize the activations
   // once into the context's scratch (Q8_0 or Q8_K, whichever the call's formats take) and run the
-  // register-tiled product; smaller batches run the matrix-vector kernel, whose workgroups take
-  // 8-row passes of their activation rows through LDS (a weight tile read from memory once per
+  // matrix product; smaller batches run the matrix-vector kernel, whose workgroups take 8-row
+  // passes of their activation rows through LDS (a weight tile read from memory once per
   // workgroup, not once per pass).
-  auto gemm_format = [&](uint32_t) { return batch >= jma::kQGemmMinBatch; };
+  const bool gemm = batch >= jma::kQGemmMinBatch;
+  char* act = nullptr;
+  char* act_scale = nullptr;
   int8_t* aq = nullptr;
   float* as = nullptr;
   int* asum = nullptr;
   set_device(ctx);
-  bool need_gemm = false;
-  std::vector<uint32_t> pass_fmts;
-  for (const QuantMatrix& m : mats) {
-    if (gemm_format(m.format)) need_gemm = true;
-    else pass_fmts.push_back(m.format);
-  }
-  if (need_gemm) {
+  if (gemm) {
     const uint64_t q_bytes = ((uint64_t)batch * cols + 255u) & ~(uint64_t)255u;
     const uint64_t s_bytes = ((uint64_t)batch * K * sizeof(float) + 255u) & ~(uint64_t)255u;
-    const uint64_t sum_bytes = kq ? (uint64_t)batch * (cols / 16u) * sizeof(int) : 0u;
-    ctx->qact.reserve(q_bytes + s_bytes + sum_bytes, ctx->stream, "projection activations");
+    ctx->qact.reserve(jma::qact_reserve_bytes((uint64_t)batch * cols), ctx->stream, "projection activations");
+    act = (char*)ctx->qact.ptr;
+    act_scale = act + jma::qact_bytes(batch, cols);
     aq = (int8_t*)ctx->qact.ptr;
     as = (float*)((char*)ctx->qact.ptr + q_bytes);
     asum = kq ? (int*)((char*)ctx->qact.ptr + q_bytes + s_bytes) : nullptr;
@@ -853,18 +850,25 @@ void quantized_matmul_impl(jmodels_attn_context* ctx, const std::vector<QuantMat
       hip_check(jma::launch_q8_k_quant(input, batch, cols, aq, as, asum, ctx->stream),
                 "activation quantization launch");
     else
-      hip_check(jma::launch_q8_0_quant(input, batch, cols, aq, as, ctx->stream),
+      hip_check(jma::launch_q8_0_quant(input, batch, cols, act, act_scale, ctx->stream),
                 "activation quantization launch");
   }
   jma::QMatPlan qp;
-  if (!pass_fmts.empty()) {
-    qp = jma::plan_qmat(pass_fmts.data(), (uint32_t)pass_fmts.size(), cols);
+  if (!gemm) {
+    std::vector<uint32_t> formats;
+    for (const QuantMatrix& m : mats) formats.push_back(m.format);
+    qp = jma::plan_qmat(formats.data(), (uint32_t)formats.size(), cols);
     require(qp.rows_per_tile > 0, JMODELS_ATTN_INVALID_SHAPE,
             "cols too large for the device projection: " + std::to_string(cols));
   }
   for (uint32_t fmt = 0; fmt <= JMODELS_ATTN_WEIGHTS_Q5_0; ++fmt) {
-    const bool gemm = gemm_format(fmt);
-    const uint32_t R = gemm ? jma::kQGemmTile : qp.rows_per_tile;
+    uint32_t fmt_rows[jma::kQMaxMatrices], count = 0;
+    for (const QuantMatrix& m : mats)
+      if (m.format == fmt) fmt_rows[count++] = m.rows;
+    if (count == 0) continue;
+    const uint32_t shape = gemm ? jma::plan_qgemm(fmt_rows, count, batch, ctx->cus) : 0u;
+    const uint32_t R = !gemm ? qp.rows_per_tile
+                       : kq ? jma::kQGemmTile : jma::qgemm_rows_w(jma::kQGemmShape[shape]);
     jma::QMatArgs a{};
     a.x = input;
     a.batch = batch;
@@ -887,14 +891,14 @@ void quantized_matmul_impl(jmodels_attn_context* ctx, const std::vector<QuantMat
       }
       out_off += (uint64_t)batch * m.rows;
     }
-    if (a.count == 0) continue;
     if (gemm) {
-      require((batch + jma::kQGemmTile - 1) / jma::kQGemmTile <= 65535u, JMODELS_ATTN_INVALID_SHAPE,
+      require((batch + 63u) / 64u <= 65535u, JMODELS_ATTN_INVALID_SHAPE,
               "batch_size too large for one projection launch: " + std::to_string(batch));
       if (kq)
         hip_check(jma::launch_qkgemm(a, fmt, tiles, aq, as, asum, ctx->stream), "quantized matmul launch");
       else
-        hip_check(jma::launch_qgemm(a, fmt, tiles, aq, as, ctx->stream), "quantized matmul launch");
+        hip_check(jma::launch_qgemm(a, fmt, shape, tiles, act, act_scale, ctx->stream),
+                  "quantized matmul launch");
     } else {
       a.group_rows = jma::qmat_group_rows(batch, qp.chunk, tiles);
       require((batch + a.group_rows - 1) / a.group_rows <= 65535u, JMODELS_ATTN_INVALID_SHAPE,

@@ -214,21 +214,23 @@ hipError_t launch_qmatvec(const QMatArgs& a, uint32_t fmt, uint32_t, hipStream_t
   return submit(stream, "qmatvec_kernel", l);
 }
 
-hipError_t launch_q8_0_quant(const float* x, uint32_t batch, uint32_t cols, int8_t* q,
-                             float* scales, hipStream_t stream) {
+hipError_t launch_q8_0_quant(const float* x, uint32_t batch, uint32_t cols, void* act, void* scales,
+                             hipStream_t stream) {
   Launch* l = new Launch();
+  const size_t rows = (size_t)qact_tiles(batch) * 32;
   add(l, x, (size_t)batch * cols * 4, "activations");
-  add(l, q, (size_t)batch * cols, "quantized activations");
-  add(l, scales, (size_t)batch * (cols / 32) * 4, "activation scales");
+  add(l, act, rows * cols * 2, "quantized activations");
+  add(l, scales, rows * (cols / 32) * 2, "activation scales");
   return submit(stream, "q8_0_quant_kernel", l);
 }
 
-hipError_t launch_qgemm(const QMatArgs& a, uint32_t fmt, uint32_t, const int8_t* aq, const float* as,
-                        hipStream_t stream) {
+hipError_t launch_qgemm(const QMatArgs& a, uint32_t fmt, uint32_t, uint32_t, const void* act,
+                        const void* act_scale, hipStream_t stream) {
   Launch* l = new Launch();
+  const size_t rows = (size_t)qact_tiles(a.batch) * 32;
   add_matrices(l, a, fmt);
-  add(l, aq, (size_t)a.batch * a.cols, "quantized activations");
-  add(l, as, (size_t)a.batch * a.blocks * 4, "activation scales");
+  add(l, act, rows * a.cols * 2, "quantized activations");
+  add(l, act_scale, rows * a.blocks * 2, "activation scales");
   return submit(stream, "qgemm_kernel", l);
 }
 

@@ -46,6 +46,7 @@ struct Buffers {
   std::vector<uint8_t*> w;
   std::vector<float*> add;
   float* x = nullptr;           // activations [batch][cols]
+  std::vector<uint16_t> act, act_scale;  // activations and scales of the 32-element products
   int8_t* aq = nullptr;         // quantized activations [batch][cols]
   float* as = nullptr;          // their scales [batch][cols / block]
   int* asum = nullptr;          // Q8_K 16-element sums [batch][cols / 16]
@@ -71,14 +72,107 @@ std::vector<M> table(const Call& c, uint32_t fmt, uint32_t R, uint32_t& tiles) {
   return ms;
 }
 
-// qgemm_kernel / qkgemm_kernel: each thread stages one weight block and one activation block per
+// qgemm_kernel: workgroups in qgemm_tile's order, each thread stages one weight block per step (rows
+// and blocks clamped to the last valid one), each wave its 1 KB pieces of the activation stage and
+// its scales; outputs in 32 x 32 tiles. Every access at its first and last byte.
+void walk_qgemm(const Call& c, uint32_t fmt, const jma::QGemmShape s, Buffers& B) {
+  const uint32_t K = c.cols / 32u, kB = jma::qgemm_rows_b(s), kW = jma::qgemm_rows_w(s);
+  const uint32_t threads = jma::qgemm_threads(s), waves = s.nb * s.nw, units = kW * 2;
+  uint32_t tiles;
+  const std::vector<M> ms = table(c, fmt, kW, tiles);
+  const uint32_t bb = jma::qmat_block_bytes(fmt), tiles_b = (c.batch + kB - 1) / kB;
+  const uint32_t total = tiles * tiles_b, btiles = jma::qact_tiles(c.batch);
+  const uint32_t pieces = kB / 32 * 2, ppw = (pieces + waves - 1) / waves;
+  std::vector<uint8_t> seen(total, 0);
+  expect(units <= threads, c.name + ": at most one staged half block per thread");
+  std::vector<uint16_t> w_lds(kW * 32), a_lds(kB * 32), c_lds(kW);
+  for (uint32_t id = 0; id < total; ++id) {
+    uint32_t tx, ty;
+    jma::qgemm_tile(id, tiles, jma::qgemm_recip(tiles), total, tx, ty);
+    expect(tx < tiles && ty < tiles_b, c.name + ": product tile in range");
+    seen[ty * tiles + tx]++;
+    uint32_t mi = 0;
+    for (uint32_t i = 1; i < ms.size(); ++i) mi = tx >= ms[i].tile0 ? i : mi;
+    const uint32_t idx = ms[mi].idx, rows = c.rows[idx];
+    const uint32_t r0 = (tx - ms[mi].tile0) * kW, b0 = ty * kB;
+    expect(r0 < rows, c.name + ": product tile past its matrix");
+    auto a_tile = [&](uint32_t i) { return std::min(b0 / 32u + i, btiles - 1u); };
+    for (uint32_t step = 0; step < (K + 3) / 4 * 4 + 3; ++step) {  // loads run three steps ahead
+      const uint64_t k = std::min(step, K - 1u);
+      std::vector<uint8_t> w_put(kW * 4, 0), a_put(pieces, 0);
+      for (uint32_t tid = 0; tid < threads; ++tid) {
+        const uint32_t su_row = tid % units / 2u, h = tid & 1u;
+        const uint64_t row = std::min(r0 + su_row, rows - 1u);
+        const uint8_t* blk = B.w[idx] + (row * K + k) * bb;
+        const uint32_t q = (fmt == 5 ? 6u : 2u) + 8u * h;
+        sink = sink + blk[0] + blk[1] + blk[q] + blk[q + 7u] + blk[fmt == 1 ? 18u + 8u * h + 7u : 5u];
+        const uint32_t slot = (su_row / 32u) * 1024u + h * 256u + (su_row % 32u) * 8u;
+        for (uint32_t i = 0; i < 2; ++i) {
+          w_lds[slot + i * 512] = 0;
+          w_lds[slot + i * 512 + 7] = 0;
+          w_put[(slot + i * 512) / 256] = 1;  // one of the 32-row runs of 8
+        }
+        c_lds[su_row] = 0;
+      }
+      for (uint32_t wv = 0; wv < waves; ++wv) {
+        for (uint32_t i = 0; i < ppw; ++i) {
+          const uint32_t p = (wv + waves * i) % pieces;
+          const uint64_t off = (uint64_t)a_tile(p / 2u) * 32u * c.cols + p % 2u * 512u + k * 1024u;
+          sink = sink + B.act[off] + B.act[off + 511];
+          a_lds[p * 512] = 0;
+          a_lds[p * 512 + 511] = 0;
+          a_put[p] = 1;
+        }
+        for (uint32_t i = 0; i < s.bt; ++i) {
+          const uint32_t t = wv / s.nw * s.bt + i;
+          sink = sink + B.act_scale[((uint64_t)a_tile(t) * K + k) * 32u + 31u] + a_lds[t * 1024 + 512 + 63 * 8 + 7];
+        }
+        for (uint32_t i = 0; i < s.wt; ++i) {
+          const uint32_t t = wv % s.nw * s.wt + i;
+          sink = sink + w_lds[t * 1024 + 512 + 63 * 8 + 7] + c_lds[t * 32 + 31];
+        }
+      }
+      for (uint32_t i = 0; i < kW * 4 / 32; ++i) expect(w_put[i] == 1, c.name + ": every weight run staged");
+      for (uint8_t n : a_put) expect(n == 1, c.name + ": every activation piece loaded");
+    }
+    for (uint32_t r = r0; r < std::min(r0 + kW, rows); ++r)
+      for (uint32_t b = b0; b < std::min(b0 + kB, c.batch); ++b) {
+        const uint64_t o = (uint64_t)b * rows + r;
+        if (c.addend_mode == 1) sink = sink + B.add[idx][r];
+        if (c.addend_mode == 2) sink = sink + B.add[idx][o];
+        B.written[ms[mi].out_off + o]++;
+      }
+  }
+  for (uint8_t n : seen) expect(n == 1, c.name + ": every product tile once");
+}
+
+// The activation quantization of the products: every element and scale of every 32-row tile once.
+void walk_quant(const Call& c, Buffers& B) {
+  const uint32_t K = c.cols / 32u, rows = jma::qact_tiles(c.batch) * 32u;
+  for (uint32_t b = 0; b < rows; ++b)
+    for (uint32_t k = 0; k < c.cols; k += 8) {
+      const uint64_t at = jma::qact_index(b, k, c.cols);
+      expect(at % 8 == 0, c.name + ": activation run aligned");
+      B.act[at]++;
+      B.act[at + 7]++;
+      if (k % 32 == 0) B.act_scale[jma::qact_scale_index(b, k / 32, K)]++;
+    }
+  for (uint64_t i = 0; i < (uint64_t)rows * c.cols; i += 8)
+    expect(B.act[i] == 1 && B.act[i + 7] == 1, c.name + ": every activation run once");
+  for (uint64_t i = 0; i < (uint64_t)rows * K; ++i)
+    expect(B.act_scale[i] == 1, c.name + ": every activation scale once");
+  const uint64_t used = jma::qact_bytes(c.batch, c.cols) + (uint64_t)rows * K * 2;
+  expect(used <= jma::qact_reserve_bytes((uint64_t)c.batch * c.cols), c.name + ": activation scratch");
+}
+
+// qkgemm_kernel: each thread stages one weight block and one activation block per
 // step (rows clamped to the last valid one and skipped past it), every thread writes 4 x 4 outputs.
 // q6gemm_kernel (Q6_K): four threads per row each stage a quarter of the 210-byte block and of the
 // 256 activation bytes into lane-major int16 stages.
 void walk_gemm(const Call& c, uint32_t fmt, Buffers& B) {
   const bool kq = jma::qmat_kquant(fmt);
   const uint32_t T = jma::kQGemmTile, KB = c.cols / jma::qmat_block_elems(fmt);
-  const uint32_t KC = kq ? 1u : jma::kQGemmKc;  // blocks staged per step
+  const uint32_t KC = 1u;  // one block staged per step
   const uint32_t per = kq ? 4u : KC;            // staging threads per row (K-quants: 4 parts)
   const uint32_t kRow = kq ? 256u + 16u : KC * 32u + 16u;
   uint32_t tiles;
@@ -244,6 +338,12 @@ void walk(const Call& c) {
   B.as = new float[(uint64_t)c.batch * K];
   B.asum = new int[(uint64_t)c.batch * (c.cols / 16u)];
   B.written.assign(c.batch * total_rows, 0);
+  if (!kq && gemm_format(c.formats[0], c.batch)) {
+    const uint64_t rows32 = (uint64_t)jma::qact_tiles(c.batch) * 32u;
+    B.act.assign(rows32 * c.cols, 0);
+    B.act_scale.assign(rows32 * K, 0);
+    walk_quant(c, B);
+  }
   std::vector<uint32_t> pass_fmts;
   for (uint32_t f : c.formats)
     if (!gemm_format(f, c.batch)) pass_fmts.push_back(f);
@@ -256,7 +356,21 @@ void walk(const Call& c) {
   for (uint32_t fmt = 0; fmt <= 5; ++fmt) {
     if (std::find(c.formats.begin(), c.formats.end(), fmt) == c.formats.end()) continue;
     if (gemm_format(fmt, c.batch)) {
-      walk_gemm(c, fmt, B);
+      if (jma::qmat_kquant(fmt)) {
+        walk_gemm(c, fmt, B);
+      } else {
+        // Every workgroup tile the planner may choose, the chosen one into the written counts.
+        std::vector<uint32_t> fmt_rows;
+        for (uint32_t i = 0; i < n; ++i)
+          if (c.formats[i] == fmt) fmt_rows.push_back(c.rows[i]);
+        const uint32_t chosen = jma::plan_qgemm(fmt_rows.data(), (uint32_t)fmt_rows.size(), c.batch, 256);
+        expect(chosen < jma::kQGemmShapes, c.name + ": product shape");
+        for (uint32_t s = 0; s < jma::kQGemmShapes; ++s) {
+          const std::vector<uint8_t> before = B.written;
+          walk_qgemm(c, fmt, jma::kQGemmShape[s], B);
+          if (s != chosen) B.written = before;
+        }
+      }
       how += " fmt " + std::to_string(fmt) + ": product;";
     } else if (qp.rows_per_tile > 0) {
       walk_pass(c, fmt, qp, B);
