@@ -280,27 +280,53 @@ constexpr uint32_t kQGemmMinBatch = 16;
 
 // Quantized activations of a product, as halves (the int8 values exactly) in the order the matrix
 // ops read them: tiles of 32 activation rows; per tile, chunks of 16 inputs, each [k half h][row]
-// [8 inputs], so the 64 lanes (32 h + row) of one operand load read 1 KB in order. Element index
-// of input k of row b:
+// [8 inputs], so the 64 lanes (32 h + row) of one operand load read 1 KB in order. Inside a run of
+// 8 the second and third of every four inputs change places, the order in which nibbles and bytes
+// of a word come out as pairs of halves. Element index of input k of row b:
 JMA_HD uint64_t qact_index(uint32_t b, uint32_t k, uint32_t cols) {
+  const uint32_t i = k % 8u, at = (i & ~3u) | ((i & 1u) << 1) | ((i >> 1) & 1u);
   return (uint64_t)(b / 32u) * 32u * cols + (uint64_t)(k / 16u) * 512u + ((k / 8u) % 2u) * 256u +
-         (b % 32u) * 8u + k % 8u;
+         (b % 32u) * 8u + at;
+}
+// The same for Q6_K weights: per 256-element block, the eight classes l of elements whose index
+// within their 32-element run is l + 8 m, m < 4; per class, the block's two 128-element halves as
+// chunks, each [run % 2][row][m / 2][run / 2][m % 2].
+JMA_HD uint64_t qact_class_index(uint32_t b, uint32_t k, uint32_t cols) {
+  const uint32_t e = k % 256u, hf = e / 128u, run = e / 32u % 4u, l = e % 8u, m = e / 8u % 4u;
+  return (uint64_t)(b / 32u) * 32u * cols + (uint64_t)(k / 256u) * 8192u + (l * 2u + hf) * 512u +
+         (run % 2u) * 256u + (b % 32u) * 8u + (m / 2u) * 4u + (run / 2u) * 2u + m % 2u;
 }
 // Scale of block blk (of K per row) of row b.
 JMA_HD uint64_t qact_scale_index(uint32_t b, uint32_t blk, uint32_t K) {
   return (uint64_t)(b / 32u) * 32u * K + (uint64_t)blk * 32u + b % 32u;
 }
+// Q8_K: sum i (of 16 elements each) of block blk, a matrix operand of 16 inputs per block.
+JMA_HD uint64_t qact_sum_index(uint32_t b, uint32_t blk, uint32_t i, uint32_t KB) {
+  return ((uint64_t)(b / 32u) * KB + blk) * 512u + (i / 8u) * 256u + (b % 32u) * 8u + i % 8u;
+}
 JMA_HD uint32_t qact_tiles(uint32_t batch) { return (batch + 31u) / 32u; }
-
 // Bytes of the activations of a batch (32-row tiles), rounded up to keep what follows aligned.
 JMA_HD uint64_t qact_bytes(uint32_t batch, uint32_t cols) {
   return ((uint64_t)qact_tiles(batch) * 32u * cols * 2u + 255u) / 256u * 256u;
 }
+// Q8_K scratch: the activations in both orders, the sums, the scales, from its start.
+struct QactKOffsets {
+  uint64_t classes, sums, scales, total;
+};
+JMA_HD QactKOffsets qact_k_offsets(uint32_t batch, uint32_t cols) {
+  QactKOffsets o;
+  const uint64_t blocks = (uint64_t)qact_tiles(batch) * (cols / 256u);
+  o.classes = qact_bytes(batch, cols);
+  o.sums = 2u * o.classes;
+  o.scales = o.sums + blocks * 1024u;
+  o.total = o.scales + blocks * 32u * 4u;
+  return o;
+}
 // Scratch to hold for calls of up to `elements` = batch x cols activations, whatever their format
 // and shape, so that a captured call no larger than an eager one before it never has to grow it:
-// rounding a batch of 16 or more up to 32 rows at most doubles it; scales and sums take at most
-// 1/4 + 1/32 of a byte per byte of int8 (Q8_K: one f32 per 256, one 16-bit sum per 16).
-JMA_HD uint64_t qact_reserve_bytes(uint64_t elements) { return elements * 4u + elements / 2u + 4096u; }
+// rounding a batch of 16 or more up to 32 rows at most doubles it (two orders of 2-byte values:
+// 8 bytes per activation); sums and scales take at most 1/4 + 1/32 of a byte more.
+JMA_HD uint64_t qact_reserve_bytes(uint64_t elements) { return elements * 8u + elements / 2u + 4096u; }
 
 // Workgroup tiles of the product: 32 bt nb activation rows x 32 wt nw weight rows on nb x nw
 // waves of bt x wt 32 x 32 tiles each, half a weight block staged per thread and step.
@@ -310,13 +336,19 @@ struct QGemmShape {
 constexpr uint32_t qgemm_rows_b(QGemmShape s) { return 32u * s.bt * s.nb; }
 constexpr uint32_t qgemm_rows_w(QGemmShape s) { return 32u * s.wt * s.nw; }
 constexpr uint32_t qgemm_threads(QGemmShape s) { return 64u * s.nb * s.nw; }
-constexpr uint32_t kQGemmTile = 64;  // K-quants
 constexpr uint32_t kQGemmShapes = 3;
 constexpr QGemmShape kQGemmShape[kQGemmShapes] = {
     {2, 2, 2, 2},  // 128 x 128
     {1, 1, 2, 2},  // 64 x 64
     {1, 1, 1, 4},  // 32 x 128
 };
+// The tile of a format: Q5_K keeps a second set of integer sums, so its large tile is 128 x 64;
+// Q6_K eight float chains per output, one 32 x 32 tile per wave (128 x 64 on eight waves).
+constexpr QGemmShape kQ5KLargeShape{2, 1, 2, 2};
+constexpr QGemmShape kQ6KShape{1, 1, 4, 2};
+JMA_HD QGemmShape qgemm_shape(uint32_t fmt, uint32_t shape) {
+  return fmt == 3 ? kQ6KShape : fmt == 4 && shape == 0 ? kQ5KLargeShape : kQGemmShape[shape];
+}
 
 // Tile (tx, ty) of workgroup `id` of a launch of `total` = tiles_w x batch tiles: the workgroups
 // of one XCD (dispatch order modulo 8) take consecutive tiles, the weight tiles fastest, so that

@@ -27,6 +27,7 @@ namespace {
 constexpr uint32_t kQThreads = 256;
 typedef short short2_t __attribute__((ext_vector_type(2)));
 typedef _Float16 half8_t __attribute__((ext_vector_type(8)));
+typedef _Float16 half2_t __attribute__((ext_vector_type(2)));
 
 template <int kCtrl>
 __device__ __forceinline__ int dpp_int(int x) {
@@ -507,6 +508,16 @@ __global__ __launch_bounds__(kQThreads) void qkmatvec_kernel(const QMatArgs a) {
 // Batches of kQGemmMinBatch activation rows and more run as matrix products on activations
 // quantized once into scratch, in the matrix ops' operand order (qact_index, qact_scale_index).
 
+// Eight int8 as halves in the order of a run of qact_index.
+__device__ __forceinline__ half8_t act_run(uint2 packed) {
+  half8_t v;
+#pragma unroll
+  for (int i = 0; i < 8; ++i)
+    v[(i & ~3) | ((i & 1) << 1) | ((i >> 1) & 1)] =
+        (_Float16)(short)(int8_t)((i < 4 ? packed.x : packed.y) >> (8 * (i & 3)));
+  return v;
+}
+
 // Q8_0 activations of the 32-element formats: a wave takes one block of 16 rows, a quad of lanes
 // per row. Rows past the batch (up to a multiple of 32) get zeros.
 __global__ __launch_bounds__(kQThreads) void q8_0_quant_kernel(const float* x, uint32_t batch,
@@ -521,10 +532,7 @@ __global__ __launch_bounds__(kQThreads) void q8_0_quant_kernel(const float* x, u
   float scale;
   int s;
   q8_0_eighth(x + (uint64_t)min(b, batch - 1u) * cols + blk * 32u + qtr * 8u, packed, scale, s);
-  half8_t v;
-#pragma unroll
-  for (int i = 0; i < 8; ++i)
-    v[i] = (_Float16)(short)(int8_t)((i < 4 ? packed.x : packed.y) >> (8 * (i & 3)));
+  half8_t v = act_run(packed);
   if (b >= batch) {
     v = half8_t{};
     scale = 0.0f;
@@ -534,416 +542,57 @@ __global__ __launch_bounds__(kQThreads) void q8_0_quant_kernel(const float* x, u
     scales[qact_scale_index(b, blk, K)] = __builtin_bit_cast(uint16_t, (_Float16)scale);
 }
 
-// Q8_K activations [batch][cols] -> int8 [batch][cols], f32 scales [batch][cols / 256] and int
-// 16-element sums [batch][cols / 16]; 32 threads per block.
+// Q8_K activations of the K-quants: a workgroup takes one 256-element block of 8 rows, 32 threads
+// a row with 8 elements each. Rows past the batch (up to a multiple of 32) get zeros. The block's
+// sixteen 16-element sums (below 2048 in magnitude, exact in f16) and its scale go beside them;
+// `classes` (null = not needed) gets the values in Q6_K's order too.
 __global__ __launch_bounds__(kQThreads) void q8_k_quant_kernel(const float* x, uint32_t batch,
-                                                               uint32_t cols, int8_t* q,
-                                                               float* scales, int* sums) {
-  const uint32_t KB = cols / 256u;
-  const uint64_t units = (uint64_t)batch * KB * 32u;
-  const uint64_t t = (uint64_t)blockIdx.x * kQThreads + threadIdx.x;
-  if (t >= units) return;  // whole blocks: units is a multiple of 32
-  const uint64_t b = t / (KB * 32u);
-  const uint32_t blk = (uint32_t)((t / 32u) % KB), part = (uint32_t)(t & 31u);
+                                                               uint32_t cols, _Float16* act,
+                                                               _Float16* classes, _Float16* sums,
+                                                               float* scales) {
+  const uint32_t KB = cols / 256u, blk = blockIdx.x % KB;
+  const uint32_t b = blockIdx.x / KB * 8u + threadIdx.x / 32u, part = threadIdx.x & 31u;
   uint2 packed;
   int s;
   float scale;
-  q8_k_part(x + b * cols + blk * 256u + part * 8u, part, packed, s, scale);
-  *(uint2*)(q + b * cols + blk * 256u + part * 8u) = packed;
-  if ((part & 1u) == 0) sums[b * (cols / 16u) + blk * 16u + part / 2u] = s;
-  if (part == 0) scales[b * KB + blk] = scale;
-}
-
-// The register-tiled product of Q4_K (FMT 2) and Q5_K (FMT 4) weights on Q8_K activations, with
-// the float order of dot_q4_k_q8_k_row_scalar / dot_q5_k_q8_k_row_scalar (RS:3410-3518): per
-// 256-element block the integer sums qsum = sum over groups of scale_g * dot_g and msum = sum of
-// min_g * (the group's two 16-element activation sums), then sum = fma(d * as, qsum, sum) and
-// sum = fma(-(dmin * as), msum, sum). Tiles of kQGemmTile x kQGemmTile outputs, 4 x 4 per thread,
-// one 256-element block staged per step: the quants as bytes (0..31), each row's 6-bit scales and
-// mins, d and dmin; the activations' bytes, scale and per-group sums. The integer arithmetic is
-// exact in narrow forms: a group's dot is at most 32 x 31 x 128 in magnitude, so scale_g * dot_g
-// is a 24-bit multiply-add, and mins (0..63) and group sums (at most 32 x 128) are 16-bit, so msum
-// is four v_dot2_i32_i16.
-template <int FMT>
-__global__ __launch_bounds__(kQThreads, 2) void qkgemm_kernel(const QMatArgs a, const int8_t* aq,
-                                                              const float* as, const int* asum) {
-  constexpr uint32_t T = kQGemmTile, kRow = 256u + 16u, kBB = FMT == 2 ? 144u : 176u;
-  __shared__ __attribute__((aligned(16))) int8_t s_w[T * kRow];
-  __shared__ __attribute__((aligned(16))) int8_t s_a[T * kRow];
-  __shared__ __attribute__((aligned(16))) int s_sc[T][8];
-  __shared__ __attribute__((aligned(16))) int16_t s_mn[T][8];
-  __shared__ __attribute__((aligned(16))) int16_t s_gs[T][8];
-  __shared__ float s_d[T], s_dm[T], s_as[T];
-  const uint32_t KB = a.blocks, cols = a.cols, batch = a.batch;
-  uint32_t mi = 0;
-  for (uint32_t i = 1; i < a.count; ++i) mi = blockIdx.x >= a.m[i].tile0 ? i : mi;
-  const uint8_t* w = a.m[mi].w;
-  float* out = a.m[mi].out;
-  const float* addend = a.m[mi].addend;
-  const uint32_t rows = a.m[mi].rows;
-  const uint32_t r0 = (blockIdx.x - a.m[mi].tile0) * T, b0 = blockIdx.y * T;
-  const uint32_t tid = threadIdx.x;
-  const uint32_t ti = tid / 16u, tj = tid % 16u;
-  // Staging: row tid / 4, part tid % 4 (groups 2 part and 2 part + 1: 64 elements).
-  const uint32_t su_row = tid / 4u, part = tid % 4u;
-  const bool w_ok = r0 + su_row < rows, a_ok = b0 + su_row < batch;
-  const uint8_t* w_row = w + (uint64_t)min(r0 + su_row, rows - 1) * KB * kBB;
-  const uint64_t arow = min(b0 + su_row, batch - 1);
-
-  float acc[4][4];
-#pragma unroll
-  for (int i = 0; i < 4; ++i)
-#pragma unroll
-    for (int j = 0; j < 4; ++j) acc[i][j] = 0.0f;
-
-  for (uint32_t kb = 0; kb < KB; ++kb) {
-    {
-      uint32_t q[16];  // 64 quant bytes: group 2 part, then 2 part + 1
-#pragma unroll
-      for (int i = 0; i < 16; ++i) q[i] = 0u;
-      if (w_ok) {
-        const uint16_t* h = (const uint16_t*)(w_row + (uint64_t)kb * kBB);
-        const uint16_t* qs = h + (FMT == 4 ? 24 : 8) + part * 16;  // 32 bytes of nibbles
-#pragma unroll
-        for (int i = 0; i < 8; ++i) {
-          const uint32_t x = (uint32_t)qs[2 * i] | ((uint32_t)qs[2 * i + 1] << 16);
-          q[i] = x & 0x0F0F0F0Fu;
-          q[8 + i] = (x >> 4) & 0x0F0F0F0Fu;
-        }
-        if constexpr (FMT == 4) {
-#pragma unroll
-          for (int i = 0; i < 8; ++i) {
-            const uint32_t qh = (uint32_t)h[8 + 2 * i] | ((uint32_t)h[9 + 2 * i] << 16);
-            q[i] |= ((qh >> (2 * part)) & 0x01010101u) << 4;
-            q[8 + i] |= ((qh >> (2 * part + 1)) & 0x01010101u) << 4;
-          }
-        }
-        if (part == 0) {
-          s_d[su_row] = f16_bits_to_float(h[0]);
-          s_dm[su_row] = f16_bits_to_float(h[1]);
-          uint32_t scb[12];
-#pragma unroll
-          for (int i = 0; i < 6; ++i) {
-            scb[2 * i] = h[2 + i] & 0xFFu;
-            scb[2 * i + 1] = h[2 + i] >> 8;
-          }
-#pragma unroll
-          for (int g = 0; g < 8; ++g) {
-            s_sc[su_row][g] = g < 4 ? (int)(scb[g] & 63u) : (int)((scb[g + 4] & 15u) | ((scb[g - 4] >> 6) << 4));
-            s_mn[su_row][g] = (int16_t)(g < 4 ? (scb[g + 4] & 63u) : ((scb[g + 4] >> 4) | ((scb[g] >> 6) << 4)));
-          }
-        }
-      } else if (part == 0) {
-        s_d[su_row] = 0.0f;
-        s_dm[su_row] = 0.0f;
-#pragma unroll
-        for (int g = 0; g < 8; ++g) {
-          s_sc[su_row][g] = 0;
-          s_mn[su_row][g] = 0;
-        }
-      }
-      uint4* dw = (uint4*)(s_w + su_row * kRow + part * 64u);
-#pragma unroll
-      for (int i = 0; i < 4; ++i) dw[i] = make_uint4(q[4 * i], q[4 * i + 1], q[4 * i + 2], q[4 * i + 3]);
-      uint4 av[4] = {make_uint4(0u, 0u, 0u, 0u), make_uint4(0u, 0u, 0u, 0u), make_uint4(0u, 0u, 0u, 0u),
-                     make_uint4(0u, 0u, 0u, 0u)};
-      int4 sm = make_int4(0, 0, 0, 0);
-      float asc = 0.0f;
-      if (a_ok) {
-        const uint4* pa = (const uint4*)(aq + arow * cols + kb * 256u + part * 64u);
-#pragma unroll
-        for (int i = 0; i < 4; ++i) av[i] = pa[i];
-        sm = *(const int4*)(asum + arow * (cols / 16u) + kb * 16u + part * 4u);
-        asc = as[arow * KB + kb];
-      }
-      uint4* da = (uint4*)(s_a + su_row * kRow + part * 64u);
-#pragma unroll
-      for (int i = 0; i < 4; ++i) da[i] = av[i];
-      s_gs[su_row][2 * part] = (int16_t)(sm.x + sm.y);
-      s_gs[su_row][2 * part + 1] = (int16_t)(sm.z + sm.w);
-      if (part == 0) s_as[su_row] = asc;
-    }
-    __syncthreads();
-    int qsum[4][4], msum[4][4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-#pragma unroll
-      for (int j = 0; j < 4; ++j) qsum[i][j] = msum[i][j] = 0;
-    for (int g = 0; g < 8; ++g) {
-      uint4 wv[4][2], avv[4][2];
-      int sc[4];
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const uint4* pw = (const uint4*)(s_w + (4u * ti + i) * kRow + g * 32u);
-        wv[i][0] = pw[0];
-        wv[i][1] = pw[1];
-        sc[i] = s_sc[4u * ti + i][g];
-        const uint4* pa = (const uint4*)(s_a + (4u * tj + i) * kRow + g * 32u);
-        avv[i][0] = pa[0];
-        avv[i][1] = pa[1];
-      }
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          int d;  // first dot in the zero-accumulator form: no register to clear
-          asm("v_dot4_i32_i8 %0, %1, %2, 0" : "=v"(d) : "v"((int)wv[i][0].x), "v"((int)avv[j][0].x));
-          d = __builtin_amdgcn_sdot4((int)wv[i][0].y, (int)avv[j][0].y, d, false);
-          d = __builtin_amdgcn_sdot4((int)wv[i][0].z, (int)avv[j][0].z, d, false);
-          d = __builtin_amdgcn_sdot4((int)wv[i][0].w, (int)avv[j][0].w, d, false);
-          d = __builtin_amdgcn_sdot4((int)wv[i][1].x, (int)avv[j][1].x, d, false);
-          d = __builtin_amdgcn_sdot4((int)wv[i][1].y, (int)avv[j][1].y, d, false);
-          d = __builtin_amdgcn_sdot4((int)wv[i][1].z, (int)avv[j][1].z, d, false);
-          d = __builtin_amdgcn_sdot4((int)wv[i][1].w, (int)avv[j][1].w, d, false);
-          qsum[i][j] += __mul24(sc[i], d);
-        }
-    }
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const uint4 m = *(const uint4*)&s_mn[4u * ti + i][0];
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const uint4 gs = *(const uint4*)&s_gs[4u * tj + j][0];
-        int t = __builtin_amdgcn_sdot2(__builtin_bit_cast(short2_t, m.x), __builtin_bit_cast(short2_t, gs.x), 0, false);
-        t = __builtin_amdgcn_sdot2(__builtin_bit_cast(short2_t, m.y), __builtin_bit_cast(short2_t, gs.y), t, false);
-        t = __builtin_amdgcn_sdot2(__builtin_bit_cast(short2_t, m.z), __builtin_bit_cast(short2_t, gs.z), t, false);
-        msum[i][j] = __builtin_amdgcn_sdot2(__builtin_bit_cast(short2_t, m.w), __builtin_bit_cast(short2_t, gs.w), t, false);
-      }
-    }
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const float wd = s_d[4u * ti + i], wdm = s_dm[4u * ti + i];
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const float asj = s_as[4u * tj + j];
-        float d, dm;
-        {
-#pragma clang fp contract(off)
-          d = wd * asj;
-          dm = wdm * asj;
-        }
-        acc[i][j] = __builtin_fmaf(d, (float)qsum[i][j], acc[i][j]);
-        acc[i][j] = __builtin_fmaf(-dm, (float)msum[i][j], acc[i][j]);
-      }
-    }
-    __syncthreads();  // the next block overwrites the stages
+  q8_k_part(x + (uint64_t)min(b, batch - 1u) * cols + blk * 256u + part * 8u, part, packed, s, scale);
+  if (b >= batch) {
+    packed = make_uint2(0u, 0u);
+    s = 0;
+    scale = 0.0f;
   }
-#pragma unroll
-  for (int j = 0; j < 4; ++j) {
-    const uint32_t b = b0 + 4u * tj + j;
-    if (b >= batch) continue;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const uint32_t r = r0 + 4u * ti + i;
-      if (r >= rows) continue;
-      const uint64_t o = (uint64_t)b * rows + r;
-      float v = acc[i][j];
-      if (a.addend_mode == 1) v = v + addend[r];
-      else if (a.addend_mode == 2) v = v + addend[o];
-      out[o] = v;
-    }
-  }
-}
-
-// The register-tiled product of Q6_K weights on Q8_K activations, with the float order of
-// dot_q6_k_q8_k_row_scalar (RS:3519-3577): per 256-element block eight integer lane sums (lane l
-// takes the elements whose index within their 32-element run is l, l + 8, l + 16 or l + 24, in
-// both 128-element halves), then lane_l = fma(d * as, isum_l, lane_l) for l = 0..7; after the last
-// block the eight lanes are added in order to 0. One block per step: each weight quant is staged
-// with its 16-element sub-block scale applied (16 bits: scale x (quant - 32)) and each activation
-// as 16 bits, both in lane-major order (int16 index 32 l + 16 half + 4 run + i / 8 for element
-// 128 half + 32 run + i), so a lane's integer sum is 16 v_dot2_i32_i16 over 64 contiguous bytes;
-// integer sums are exact in any order. Tiles of kQGemmTile x kQGemmTile outputs, 4 x 4 per thread,
-// each output with its eight lane chains.
-__global__ __launch_bounds__(kQThreads, 2) void q6gemm_kernel(const QMatArgs a, const int8_t* aq,
-                                                              const float* as) {
-  constexpr uint32_t T = kQGemmTile, kRow = 256u + 8u, kBB = 210u;  // int16 per staged row
-  __shared__ __attribute__((aligned(16))) int16_t s_w[T * kRow];
-  __shared__ __attribute__((aligned(16))) int16_t s_a[T * kRow];
-  __shared__ float s_d[T], s_as[T];
-  const uint32_t KB = a.blocks, cols = a.cols, batch = a.batch;
-  uint32_t mi = 0;
-  for (uint32_t i = 1; i < a.count; ++i) mi = blockIdx.x >= a.m[i].tile0 ? i : mi;
-  const uint8_t* w = a.m[mi].w;
-  float* out = a.m[mi].out;
-  const float* addend = a.m[mi].addend;
-  const uint32_t rows = a.m[mi].rows;
-  const uint32_t r0 = (blockIdx.x - a.m[mi].tile0) * T, b0 = blockIdx.y * T;
-  const uint32_t tid = threadIdx.x;
-  const uint32_t ti = tid / 16u, tj = tid % 16u;
-  // Staging: row tid / 4, part tid % 4 = 128-element half (part / 2) and elements i0 .. i0 + 15 of
-  // its four 32-element runs (i0 = 16 (part % 2)), which land in dword (8 half + 2 run + part % 2)
-  // of each lane's 16.
-  const uint32_t su_row = tid / 4u, part = tid % 4u, half = part >> 1, i0 = (part & 1u) * 16u;
-  const bool w_ok = r0 + su_row < rows, a_ok = b0 + su_row < batch;
-  const uint8_t* w_row = w + (uint64_t)min(r0 + su_row, rows - 1) * KB * kBB;
-  const uint64_t arow = min(b0 + su_row, batch - 1);
-  uint32_t* const sw_row = (uint32_t*)(s_w + su_row * kRow) + 8u * half + (part & 1u);
-  uint32_t* const sa_row = (uint32_t*)(s_a + su_row * kRow) + 8u * half + (part & 1u);
-
-  float acc[4][4][8];
-#pragma unroll
-  for (int i = 0; i < 4; ++i)
-#pragma unroll
-    for (int j = 0; j < 4; ++j)
-#pragma unroll
-      for (int l = 0; l < 8; ++l) acc[i][j][l] = 0.0f;
-
-  // 16 bytes at a 2-byte aligned address, as four words.
-  auto load16 = [](const uint8_t* p, uint32_t (&x)[4]) {
-    const uint16_t* h = (const uint16_t*)p;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) x[i] = (uint32_t)h[2 * i] | ((uint32_t)h[2 * i + 1] << 16);
+  *(half8_t*)(act + qact_index(b, blk * 256u + part * 8u, cols)) = act_run(packed);
+  if ((part & 1u) == 0) sums[qact_sum_index(b, blk, part / 2u, KB)] = (_Float16)(short)s;
+  if (part == 0) scales[qact_scale_index(b, blk, KB)] = scale;
+  if (classes == nullptr) return;
+  // The four lanes of a quad hold elements l, l + 8, l + 16, l + 24 of one 32-element run for every
+  // class l: lane m takes classes 2 m and 2 m + 1, bytes 2 m and 2 m + 1 of all four lanes.
+  const uint32_t m = part & 3u, sel = (m & 1u) ? 16u : 0u;
+  half2_t lo[2], hi[2];
+  auto take = [&](auto from) {
+    constexpr int f = decltype(from)::value, ctrl = f * 0x55;  // quad_perm [f, f, f, f]
+    const uint32_t px = (uint32_t)dpp_int<ctrl>((int)packed.x), py = (uint32_t)dpp_int<ctrl>((int)packed.y);
+    const uint32_t two = (m < 2u ? px : py) >> sel;
+    lo[f / 2][f % 2] = (_Float16)(short)(int8_t)two;
+    hi[f / 2][f % 2] = (_Float16)(short)(int8_t)(two >> 8);
   };
-  // Byte t of four words.
-  auto byte_of = [](const uint32_t (&x)[4], int t) -> uint32_t { return (x[t >> 2] >> (8 * (t & 3))) & 0xFFu; };
-
-  for (uint32_t kb = 0; kb < KB; ++kb) {
-    {
-      // Weights: ql bytes i0.. of both 32-byte runs of this half, qh bytes i0.., the four
-      // sub-block scales of runs 0..3 (scale index 8 half + i0 / 16 + 2 run), d.
-      uint32_t la[4] = {0u, 0u, 0u, 0u}, lb[4] = {0u, 0u, 0u, 0u}, hb[4] = {0u, 0u, 0u, 0u};
-      int sc[4] = {0, 0, 0, 0};
-      if (w_ok) {
-        const uint8_t* blk = w_row + (uint64_t)kb * kBB;
-        load16(blk + 64u * half + i0, la);
-        load16(blk + 64u * half + 32u + i0, lb);
-        load16(blk + 128u + 32u * half + i0, hb);
-        const uint16_t* sch = (const uint16_t*)(blk + 192u + 8u * half);  // scales 8 half .. + 7
-        uint32_t s8[4];
+  take(std::integral_constant<int, 0>{});
+  take(std::integral_constant<int, 1>{});
+  take(std::integral_constant<int, 2>{});
+  take(std::integral_constant<int, 3>{});
+  const uint32_t e = blk * 256u + part / 4u * 32u + 2u * m;  // element 2 m of the run: class 2 m
 #pragma unroll
-        for (int i = 0; i < 4; ++i) s8[i] = sch[i];
-#pragma unroll
-        for (int run = 0; run < 4; ++run) {
-          // scale byte i0 / 16 + 2 run: word run, low byte when i0 = 0, high byte otherwise
-          const uint32_t b = (s8[run] >> (i0 == 0u ? 0 : 8)) & 0xFFu;
-          sc[run] = (int)(int8_t)b;
-        }
-        if (part == 0) s_d[su_row] = f16_bits_to_float(((const uint16_t*)blk)[104]);
-      } else if (part == 0) {
-        s_d[su_row] = 0.0f;
-      }
-      // Element i0 + t of run `run`: the low nibble of la (runs 0, 2: low / high nibble) or lb
-      // (runs 1, 3), the high bits 2 run of hb; elements t and t + 8 share a lane and fill its
-      // dword's low and high halves.
-#pragma unroll
-      for (int run = 0; run < 4; ++run) {
-        const uint32_t(&lo)[4] = (run & 1) ? lb : la;
-        const int shift = (run >> 1) * 4;
-#pragma unroll
-        for (int l = 0; l < 8; ++l) {
-          int v[2];
-#pragma unroll
-          for (int e = 0; e < 2; ++e) {
-            const int t = l + 8 * e;
-            const int q = (int)(((byte_of(lo, t) >> shift) & 15u) | (((byte_of(hb, t) >> (2 * run)) & 3u) << 4)) - 32;
-            v[e] = w_ok ? sc[run] * q : 0;
-          }
-          sw_row[16 * l + 2 * run] = ((uint32_t)v[0] & 0xFFFFu) | ((uint32_t)v[1] << 16);
-        }
-      }
-      // Activations: bytes i0 .. i0 + 15 of each 32-element run of this half.
-      uint4 av[4] = {make_uint4(0u, 0u, 0u, 0u), make_uint4(0u, 0u, 0u, 0u), make_uint4(0u, 0u, 0u, 0u),
-                     make_uint4(0u, 0u, 0u, 0u)};
-      float asc = 0.0f;
-      if (a_ok) {
-        const int8_t* pa = aq + arow * cols + kb * 256u + 128u * half + i0;
-#pragma unroll
-        for (int run = 0; run < 4; ++run) av[run] = *(const uint4*)(pa + 32u * run);
-        asc = as[arow * KB + kb];
-      }
-#pragma unroll
-      for (int run = 0; run < 4; ++run) {
-        const uint32_t x[4] = {av[run].x, av[run].y, av[run].z, av[run].w};
-#pragma unroll
-        for (int l = 0; l < 8; ++l) {
-          const int v0 = (int)(int8_t)byte_of(x, l), v1 = (int)(int8_t)byte_of(x, l + 8);
-          sa_row[16 * l + 2 * run] = ((uint32_t)v0 & 0xFFFFu) | ((uint32_t)v1 << 16);
-        }
-      }
-      if (part == 0) s_as[su_row] = asc;
-    }
-    __syncthreads();
-    float dd[4][4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-#pragma clang fp contract(off)
-        dd[i][j] = s_d[4u * ti + i] * s_as[4u * tj + j];
-      }
-#pragma unroll
-    for (int l = 0; l < 8; ++l) {
-      int isum[4][4];
-#pragma unroll
-      for (int qd = 0; qd < 4; ++qd) {  // lane l's 16 dwords, four at a time
-        uint4 wv[4], avv[4];
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          wv[i] = *(const uint4*)(s_w + (4u * ti + i) * kRow + 32u * l + 8u * qd);
-          avv[i] = *(const uint4*)(s_a + (4u * tj + i) * kRow + 32u * l + 8u * qd);
-        }
-#pragma unroll
-        for (int i = 0; i < 4; ++i)
-#pragma unroll
-          for (int j = 0; j < 4; ++j) {
-            int d;
-            if (qd == 0)  // the lane's first dot in the zero-accumulator form: no register to clear
-              asm("v_dot2_i32_i16 %0, %1, %2, 0" : "=v"(d) : "v"(wv[i].x), "v"(avv[j].x));
-            else
-              d = __builtin_amdgcn_sdot2(__builtin_bit_cast(short2_t, wv[i].x), __builtin_bit_cast(short2_t, avv[j].x), isum[i][j], false);
-            d = __builtin_amdgcn_sdot2(__builtin_bit_cast(short2_t, wv[i].y), __builtin_bit_cast(short2_t, avv[j].y), d, false);
-            d = __builtin_amdgcn_sdot2(__builtin_bit_cast(short2_t, wv[i].z), __builtin_bit_cast(short2_t, avv[j].z), d, false);
-            d = __builtin_amdgcn_sdot2(__builtin_bit_cast(short2_t, wv[i].w), __builtin_bit_cast(short2_t, avv[j].w), d, false);
-            isum[i][j] = d;
-          }
-      }
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int j = 0; j < 4; ++j) acc[i][j][l] = __builtin_fmaf(dd[i][j], (float)isum[i][j], acc[i][j][l]);
-    }
-    __syncthreads();  // the next block overwrites the stages
-  }
-#pragma unroll
-  for (int j = 0; j < 4; ++j) {
-    const uint32_t b = b0 + 4u * tj + j;
-    if (b >= batch) continue;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const uint32_t r = r0 + 4u * ti + i;
-      if (r >= rows) continue;
-      const uint64_t o = (uint64_t)b * rows + r;
-      float v = 0.0f;
-#pragma unroll
-      for (int l = 0; l < 8; ++l) v = v + acc[i][j][l];
-      if (a.addend_mode == 1) v = v + addend[r];
-      else if (a.addend_mode == 2) v = v + addend[o];
-      out[o] = v;
-    }
+  for (uint32_t i = 0; i < 2; ++i) {
+    *(half2_t*)(classes + qact_class_index(b, e + 16u * i, cols)) = lo[i];
+    *(half2_t*)(classes + qact_class_index(b, e + 1u + 16u * i, cols)) = hi[i];
   }
 }
 
-hipError_t launch_q8_k_quant(const float* x, uint32_t batch, uint32_t cols, int8_t* q,
-                             float* scales, int* sums, hipStream_t stream) {
-  const uint64_t units = (uint64_t)batch * (cols / 256u) * 32u;
-  const uint32_t blocks = (uint32_t)((units + kQThreads - 1) / kQThreads);
+hipError_t launch_q8_k_quant(const float* x, uint32_t batch, uint32_t cols, void* act, void* classes,
+                             void* sums, void* scales, hipStream_t stream) {
+  const uint32_t blocks = qact_tiles(batch) * 4u * (cols / 256u);
   hipLaunchKernelGGL(q8_k_quant_kernel, dim3(blocks), dim3(kQThreads), 0, stream, x, batch, cols,
-                     q, scales, sums);
-  return hipGetLastError();
-}
-
-hipError_t launch_qkgemm(const QMatArgs& a, uint32_t fmt, uint32_t tiles, const int8_t* aq,
-                         const float* as, const int* asum, hipStream_t stream) {
-  const dim3 grid(tiles, (a.batch + kQGemmTile - 1) / kQGemmTile);
-  if (fmt == 2)
-    hipLaunchKernelGGL(qkgemm_kernel<2>, grid, dim3(kQThreads), 0, stream, a, aq, as, asum);
-  else if (fmt == 4)
-    hipLaunchKernelGGL(qkgemm_kernel<4>, grid, dim3(kQThreads), 0, stream, a, aq, as, asum);
-  else if (fmt == 3)
-    hipLaunchKernelGGL(q6gemm_kernel, grid, dim3(kQThreads), 0, stream, a, aq, as);
-  else
-    return hipErrorInvalidValue;
+                     (_Float16*)act, (_Float16*)classes, (_Float16*)sums, (float*)scales);
   return hipGetLastError();
 }
 

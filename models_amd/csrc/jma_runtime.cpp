@@ -833,21 +833,17 @@ void quantized_matmul_impl(jmodels_attn_context* ctx, const std::vector<QuantMat
   const bool gemm = batch >= jma::kQGemmMinBatch;
   char* act = nullptr;
   char* act_scale = nullptr;
-  int8_t* aq = nullptr;
-  float* as = nullptr;
-  int* asum = nullptr;
+  const jma::QactKOffsets ko = jma::qact_k_offsets(batch, cols);
   set_device(ctx);
   if (gemm) {
-    const uint64_t q_bytes = ((uint64_t)batch * cols + 255u) & ~(uint64_t)255u;
-    const uint64_t s_bytes = ((uint64_t)batch * K * sizeof(float) + 255u) & ~(uint64_t)255u;
     ctx->qact.reserve(jma::qact_reserve_bytes((uint64_t)batch * cols), ctx->stream, "projection activations");
     act = (char*)ctx->qact.ptr;
-    act_scale = act + jma::qact_bytes(batch, cols);
-    aq = (int8_t*)ctx->qact.ptr;
-    as = (float*)((char*)ctx->qact.ptr + q_bytes);
-    asum = kq ? (int*)((char*)ctx->qact.ptr + q_bytes + s_bytes) : nullptr;
+    act_scale = act + (kq ? ko.scales : jma::qact_bytes(batch, cols));
+    bool q6 = false;
+    for (const QuantMatrix& m : mats) q6 |= m.format == JMODELS_ATTN_WEIGHTS_Q6_K;
     if (kq)
-      hip_check(jma::launch_q8_k_quant(input, batch, cols, aq, as, asum, ctx->stream),
+      hip_check(jma::launch_q8_k_quant(input, batch, cols, act, q6 ? act + ko.classes : nullptr,
+                                       act + ko.sums, act_scale, ctx->stream),
                 "activation quantization launch");
     else
       hip_check(jma::launch_q8_0_quant(input, batch, cols, act, act_scale, ctx->stream),
@@ -867,8 +863,7 @@ void quantized_matmul_impl(jmodels_attn_context* ctx, const std::vector<QuantMat
       if (m.format == fmt) fmt_rows[count++] = m.rows;
     if (count == 0) continue;
     const uint32_t shape = gemm ? jma::plan_qgemm(fmt_rows, count, batch, ctx->cus) : 0u;
-    const uint32_t R = !gemm ? qp.rows_per_tile
-                       : kq ? jma::kQGemmTile : jma::qgemm_rows_w(jma::kQGemmShape[shape]);
+    const uint32_t R = gemm ? jma::qgemm_rows_w(jma::qgemm_shape(fmt, shape)) : qp.rows_per_tile;
     jma::QMatArgs a{};
     a.x = input;
     a.batch = batch;
@@ -895,7 +890,9 @@ void quantized_matmul_impl(jmodels_attn_context* ctx, const std::vector<QuantMat
       require((batch + 63u) / 64u <= 65535u, JMODELS_ATTN_INVALID_SHAPE,
               "batch_size too large for one projection launch: " + std::to_string(batch));
       if (kq)
-        hip_check(jma::launch_qkgemm(a, fmt, tiles, aq, as, asum, ctx->stream), "quantized matmul launch");
+        hip_check(jma::launch_qkgemm(a, fmt, shape, tiles, fmt == JMODELS_ATTN_WEIGHTS_Q6_K ? act + ko.classes : act,
+                                     act + ko.sums, act_scale, ctx->stream),
+                  "quantized matmul launch");
       else
         hip_check(jma::launch_qgemm(a, fmt, shape, tiles, act, act_scale, ctx->stream),
                   "quantized matmul launch");

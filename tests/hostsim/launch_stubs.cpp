@@ -234,23 +234,26 @@ hipError_t launch_qgemm(const QMatArgs& a, uint32_t fmt, uint32_t, uint32_t, con
   return submit(stream, "qgemm_kernel", l);
 }
 
-hipError_t launch_q8_k_quant(const float* x, uint32_t batch, uint32_t cols, int8_t* q,
-                             float* scales, int* sums, hipStream_t stream) {
+hipError_t launch_q8_k_quant(const float* x, uint32_t batch, uint32_t cols, void* act, void* classes,
+                             void* sums, void* scales, hipStream_t stream) {
   Launch* l = new Launch();
+  const size_t rows = (size_t)qact_tiles(batch) * 32;
   add(l, x, (size_t)batch * cols * 4, "activations");
-  add(l, q, (size_t)batch * cols, "quantized activations");
-  add(l, scales, (size_t)batch * (cols / 256) * 4, "activation scales");
-  add(l, sums, (size_t)batch * (cols / 16) * 4, "activation sums");
+  add(l, act, rows * cols * 2, "quantized activations");
+  if (classes) add(l, classes, rows * cols * 2, "quantized activations in class order");
+  add(l, sums, rows * (cols / 16) * 2, "activation sums");
+  add(l, scales, rows * (cols / 256) * 4, "activation scales");
   return submit(stream, "q8_k_quant_kernel", l);
 }
 
-hipError_t launch_qkgemm(const QMatArgs& a, uint32_t fmt, uint32_t, const int8_t* aq, const float* as,
-                         const int* asum, hipStream_t stream) {
+hipError_t launch_qkgemm(const QMatArgs& a, uint32_t fmt, uint32_t, uint32_t, const void* act,
+                         const void* sums, const void* scales, hipStream_t stream) {
   Launch* l = new Launch();
+  const size_t rows = (size_t)qact_tiles(a.batch) * 32;
   add_matrices(l, a, fmt);
-  add(l, aq, (size_t)a.batch * a.cols, "quantized activations");
-  add(l, as, (size_t)a.batch * a.blocks * 4, "activation scales");
-  if (fmt != 3) add(l, asum, (size_t)a.batch * (a.cols / 16) * 4, "activation sums");
+  add(l, act, rows * a.cols * 2, "quantized activations");
+  if (fmt != 3) add(l, sums, rows * (a.cols / 16) * 2, "activation sums");
+  add(l, scales, rows * a.blocks * 4, "activation scales");
   return submit(stream, "qkgemm_kernel", l);
 }
 

@@ -46,10 +46,9 @@ struct Buffers {
   std::vector<uint8_t*> w;
   std::vector<float*> add;
   float* x = nullptr;           // activations [batch][cols]
-  std::vector<uint16_t> act, act_scale;  // activations and scales of the 32-element products
-  int8_t* aq = nullptr;         // quantized activations [batch][cols]
-  float* as = nullptr;          // their scales [batch][cols / block]
-  int* asum = nullptr;          // Q8_K 16-element sums [batch][cols / 16]
+  // quantized activations, their scales and (Q8_K) the values in class order and the sums
+  std::vector<uint16_t> act, act_scale, act_class, act_sum;
+  std::vector<float> act_scale_k;
   std::vector<uint8_t> written;  // per output element
 };
 
@@ -153,109 +152,120 @@ void walk_quant(const Call& c, Buffers& B) {
     for (uint32_t k = 0; k < c.cols; k += 8) {
       const uint64_t at = jma::qact_index(b, k, c.cols);
       expect(at % 8 == 0, c.name + ": activation run aligned");
-      B.act[at]++;
-      B.act[at + 7]++;
+      for (uint32_t i = 0; i < 8; ++i) B.act[jma::qact_index(b, k + i, c.cols)]++;
       if (k % 32 == 0) B.act_scale[jma::qact_scale_index(b, k / 32, K)]++;
     }
   for (uint64_t i = 0; i < (uint64_t)rows * c.cols; i += 8)
-    expect(B.act[i] == 1 && B.act[i + 7] == 1, c.name + ": every activation run once");
+    expect(B.act[i] == 1 && B.act[i + 3] == 1 && B.act[i + 7] == 1, c.name + ": every activation run once");
   for (uint64_t i = 0; i < (uint64_t)rows * K; ++i)
     expect(B.act_scale[i] == 1, c.name + ": every activation scale once");
   const uint64_t used = jma::qact_bytes(c.batch, c.cols) + (uint64_t)rows * K * 2;
   expect(used <= jma::qact_reserve_bytes((uint64_t)c.batch * c.cols), c.name + ": activation scratch");
 }
 
-// qkgemm_kernel: each thread stages one weight block and one activation block per
-// step (rows clamped to the last valid one and skipped past it), every thread writes 4 x 4 outputs.
-// q6gemm_kernel (Q6_K): four threads per row each stage a quarter of the 210-byte block and of the
-// 256 activation bytes into lane-major int16 stages.
-void walk_gemm(const Call& c, uint32_t fmt, Buffers& B) {
-  const bool kq = jma::qmat_kquant(fmt);
-  const uint32_t T = jma::kQGemmTile, KB = c.cols / jma::qmat_block_elems(fmt);
-  const uint32_t KC = 1u;  // one block staged per step
-  const uint32_t per = kq ? 4u : KC;            // staging threads per row (K-quants: 4 parts)
-  const uint32_t kRow = kq ? 256u + 16u : KC * 32u + 16u;
+// qkgemm_kernel (Q4_K, Q5_K) and q6gemm_kernel (Q6_K): as walk_qgemm, a step one 32-element group
+// (or class) of a block; the block's header, quants, sums and scales at their first and last bytes.
+void walk_qkgemm(const Call& c, uint32_t fmt, const jma::QGemmShape s, Buffers& B) {
+  const uint32_t KB = c.cols / 256u, kB = jma::qgemm_rows_b(s), kW = jma::qgemm_rows_w(s);
+  const uint32_t threads = jma::qgemm_threads(s), waves = s.nb * s.nw;
+  const bool q6 = fmt == 3;
   uint32_t tiles;
-  const std::vector<M> ms = table(c, fmt, T, tiles);
-  const uint32_t bb = jma::qmat_block_bytes(fmt);
-  const uint32_t gy = (c.batch + T - 1) / T;
-  expect(gy <= 65535u, c.name + ": product grid rows");
-  int8_t* lds = new int8_t[T * kRow];
-  constexpr uint32_t kRow6 = 256u + 8u;  // q6gemm_kernel's int16 per staged row
-  int16_t* lds16 = new int16_t[T * kRow6];
-  for (uint32_t bx = 0; bx < tiles; ++bx) {
+  const std::vector<M> ms = table(c, fmt, kW, tiles);
+  const uint32_t bb = jma::qmat_block_bytes(fmt), tiles_b = (c.batch + kB - 1) / kB;
+  const uint32_t total = tiles * tiles_b, btiles = jma::qact_tiles(c.batch);
+  const uint32_t pieces = kB / 32 * 2, ppw = (pieces + waves - 1) / waves;
+  const uint32_t scale_pieces = (kB + 63) / 64;
+  const std::vector<uint16_t>& act = q6 ? B.act_class : B.act;
+  std::vector<uint8_t> seen(total, 0);
+  std::vector<uint16_t> w_lds(kW * (q6 ? 64 : 32)), a_lds(kB * 32), s_lds(kW * 16);
+  std::vector<float> as_lds(scale_pieces * 64), d_lds(kW);
+  if (q6) expect(threads == kW * 8 && pieces == waves, c.name + ": Q6_K staging");
+  else expect(kW * 2 <= threads, c.name + ": at most one staged half block per thread");
+  for (uint32_t id = 0; id < total; ++id) {
+    uint32_t tx, ty;
+    jma::qgemm_tile(id, tiles, jma::qgemm_recip(tiles), total, tx, ty);
+    expect(tx < tiles && ty < tiles_b, c.name + ": product tile in range");
+    seen[ty * tiles + tx]++;
     uint32_t mi = 0;
-    for (uint32_t i = 1; i < ms.size(); ++i) mi = bx >= ms[i].tile0 ? i : mi;
+    for (uint32_t i = 1; i < ms.size(); ++i) mi = tx >= ms[i].tile0 ? i : mi;
     const uint32_t idx = ms[mi].idx, rows = c.rows[idx];
-    const uint32_t r0 = (bx - ms[mi].tile0) * T;
+    const uint32_t r0 = (tx - ms[mi].tile0) * kW, b0 = ty * kB;
     expect(r0 < rows, c.name + ": product tile past its matrix");
-    for (uint32_t by = 0; by < gy; ++by) {
-      const uint32_t b0 = by * T;
-      for (uint32_t tid = 0; tid < 256; ++tid) {
-        const uint32_t su_row = tid / per, su = tid % per;
-        const bool w_ok = r0 + su_row < rows, a_ok = b0 + su_row < c.batch;
-        const uint64_t wrow = std::min(r0 + su_row, rows - 1), arow = std::min(b0 + su_row, c.batch - 1);
-        if (fmt == 3) {  // q6gemm_kernel: int16 stages of kRow6 halves per row
-          const uint32_t half = su >> 1, i0 = (su & 1u) * 16u;
-          for (uint32_t k = 0; k < KB; ++k) {
-            const uint64_t blk = (wrow * KB + k) * bb;
-            if (w_ok) {
-              for (uint32_t off : {64u * half + i0, 64u * half + 32u + i0, 128u + 32u * half + i0})
-                sink = sink + B.w[idx][blk + off] + B.w[idx][blk + off + 15u];
-              sink = sink + B.w[idx][blk + 192u + 8u * half] + B.w[idx][blk + 192u + 8u * half + 7u];
-              if (su == 0) sink = sink + B.w[idx][blk + 208u] + B.w[idx][blk + 209u];
-            }
-            if (a_ok) {
-              for (uint32_t run = 0; run < 4; ++run) {
-                const uint64_t a0 = arow * c.cols + k * 256u + 128u * half + i0 + 32u * run;
-                sink = sink + B.aq[a0] + B.aq[a0 + 15u];
-              }
-              sink = sink + B.as[arow * KB + k];
-            }
-            for (uint32_t l = 0; l < 8; ++l)
-              for (uint32_t run = 0; run < 4; ++run) {
-                const uint32_t dw = su_row * (kRow6 / 2u) + 8u * half + (su & 1u) + 16u * l + 2u * run;
-                lds16[2 * dw] = 0;
-                lds16[2 * dw + 1] = 0;
-              }
+    auto a_tile = [&](uint32_t i) { return std::min(b0 / 32u + i, btiles - 1u); };
+    for (uint32_t kbx = 0; kbx <= KB; ++kbx) {  // loads run up to one block ahead
+      const uint64_t kb = std::min(kbx, KB - 1u);
+      std::vector<uint8_t> w_put(kW * (q6 ? 16 : 4), 0);
+      for (uint32_t tid = 0; tid < threads; ++tid) {
+        const uint32_t su_row = q6 ? tid / 8u : tid % (kW * 2) / 2u;
+        const uint8_t* blk = B.w[idx] + ((uint64_t)std::min(r0 + su_row, rows - 1u) * KB + kb) * bb;
+        if (q6) {
+          const uint32_t hf = tid >> 2 & 1u, rr = tid >> 1 & 1u, sp = tid & 1u;
+          const uint32_t ql = 64u * hf + 32u * rr + 16u * sp, qh = 128u + 32u * hf + 16u * sp;
+          sink = sink + blk[ql] + blk[ql + 15u] + blk[qh] + blk[qh + 15u] + blk[192u + 8u * hf] + blk[199u + 8u * hf] + blk[209];
+          const uint32_t slot = (su_row / 32u) * 2048u + hf * 512u + rr * 256u + (su_row % 32u) * 8u + sp * 4u;
+          for (uint32_t o = 0; o < 2; ++o) {
+            w_lds[slot + o * 1024u + 3u] = 0;
+            w_put[(slot + o * 1024u) / 4u]++;
           }
-          const uint32_t ti = tid / 16, tj = tid % 16;
-          for (uint32_t i = 0; i < 4; ++i)
-            for (uint32_t l = 0; l < 8; ++l)
-              sink = sink + lds16[(4 * ti + i) * kRow6 + 32u * l + 31u] + lds16[(4 * tj + i) * kRow6 + 32u * l];
+        } else {
+          const uint32_t h = tid & 1u, q = fmt == 4 ? 48u : 16u;
+          sink = sink + blk[0] + blk[15];
+          for (uint32_t p = 0; p < 4; ++p) sink = sink + blk[q + 32u * p + 8u * h] + blk[q + 32u * p + 16u + 8u * h + 7u];
+          if (fmt == 4) sink = sink + blk[16u + 8u * h] + blk[32u + 8u * h + 7u];
+          const uint32_t slot = (su_row / 32u) * 1024u + h * 256u + (su_row % 32u) * 8u;
+          w_lds[slot + 7u] = w_lds[slot + 512u + 7u] = 0;
+          w_put[slot / 8u] = w_put[(slot + 512u) / 8u] = 1;
+          s_lds[(su_row / 32u) * 512u + h * 256u + (su_row % 32u) * 8u + 7u] = 0;
         }
-        for (uint32_t k0 = 0; fmt != 3 && k0 < KB; k0 += KC) {
-          const uint32_t k = kq ? k0 : k0 + su;
-          if (k < KB && w_ok) sink = sink + B.w[idx][(wrow * KB + k) * bb] + B.w[idx][(wrow * KB + k) * bb + bb - 1];
-          if (k < KB && a_ok) {
-            const uint64_t a0 = arow * c.cols + k * (kq ? 256u : 32u) + (kq ? su * 64u : 0u);
-            sink = sink + B.aq[a0] + B.aq[a0 + (kq ? 63u : 31u)] + B.as[arow * KB + k];
-            if (kq) sink = sink + B.asum[arow * (c.cols / 16u) + k * 16u + su * 4u + 3u];
-          }
-          const uint32_t l0 = su_row * kRow + (kq ? su * 64u : su * 32u);
-          lds[l0] = 0;
-          lds[l0 + (kq ? 63u : 31u)] = 0;
-        }
-        const uint32_t ti = tid / 16, tj = tid % 16;
-        for (uint32_t i = 0; fmt != 3 && i < 4; ++i)
-          sink = sink + lds[(4 * ti + i) * kRow + (kq ? 255u : (KC - 1) * 32u + 31u)] + lds[(4 * tj + i) * kRow];
-        for (uint32_t j = 0; j < 4; ++j) {
-          const uint32_t b = b0 + 4 * tj + j;
-          if (b >= c.batch) continue;
-          for (uint32_t i = 0; i < 4; ++i) {
-            const uint32_t r = r0 + 4 * ti + i;
-            if (r >= rows) continue;
-            const uint64_t o = (uint64_t)b * rows + r;
-            if (c.addend_mode == 1) sink = sink + B.add[idx][r];
-            if (c.addend_mode == 2) sink = sink + B.add[idx][o];
-            B.written[ms[mi].out_off + o]++;
-          }
-        }
+        d_lds[su_row] = 0;
       }
+      for (uint32_t i = 0; i < (q6 ? kW * 16u : kW * 4u); ++i) expect(w_put[i] == 1, c.name + ": every weight run staged once");
+      for (uint32_t g = 0; g < 8; ++g)
+        for (uint32_t wv = 0; wv < waves; ++wv)
+          for (uint32_t i = 0; i < ppw; ++i) {
+            const uint32_t p = (wv + waves * i) % pieces;
+            const uint64_t off = (uint64_t)a_tile(p / 2u) * 32u * c.cols + p % 2u * 512u + (kb * 8u + g) * 1024u;
+            sink = sink + act[off] + act[off + 511];
+            a_lds[p * 512 + 511] = 0;
+          }
+      for (uint32_t i = 0; i < scale_pieces; ++i)
+        for (uint32_t h = 0; h < 2; ++h) {
+          sink = sink + B.act_scale_k[((uint64_t)a_tile(2u * i + h) * KB + kb) * 32u + 31u];
+          as_lds[64 * i + 32 * h + 31] = 0;
+        }
+      for (uint32_t t = 0; t < kB / 32 && !q6; ++t) sink = sink + B.act_sum[((uint64_t)a_tile(t) * KB + kb) * 512u + 511u];
     }
+    for (uint32_t r = r0; r < std::min(r0 + kW, rows); ++r)
+      for (uint32_t b = b0; b < std::min(b0 + kB, c.batch); ++b) {
+        const uint64_t o = (uint64_t)b * rows + r;
+        if (c.addend_mode == 1) sink = sink + B.add[idx][r];
+        if (c.addend_mode == 2) sink = sink + B.add[idx][o];
+        B.written[ms[mi].out_off + o]++;
+      }
   }
-  delete[] lds;
-  delete[] lds16;
+  for (uint8_t n : seen) expect(n == 1, c.name + ": every product tile once");
+}
+
+// q8_k_quant_kernel: every value in both orders, sum and scale of every 32-row tile once.
+void walk_quant_k(const Call& c, Buffers& B) {
+  const uint32_t KB = c.cols / 256u, rows = jma::qact_tiles(c.batch) * 32u;
+  for (uint32_t b = 0; b < rows; ++b)
+    for (uint32_t k = 0; k < c.cols; ++k) {
+      B.act[jma::qact_index(b, k, c.cols)]++;
+      B.act_class[jma::qact_class_index(b, k, c.cols)]++;
+      if (k % 16 == 0) B.act_sum[jma::qact_sum_index(b, k / 256u, k % 256u / 16u, KB)]++;
+      if (k % 256 == 0) B.act_scale_k[jma::qact_scale_index(b, k / 256u, KB)]++;
+    }
+  bool once = true;
+  for (uint64_t i = 0; i < (uint64_t)rows * c.cols; ++i) once &= B.act[i] == 1 && B.act_class[i] == 1;
+  for (uint64_t i = 0; i < (uint64_t)rows * KB * 16u; ++i) once &= B.act_sum[i] == 1;
+  for (uint64_t i = 0; i < (uint64_t)rows * KB; ++i) once &= B.act_scale_k[i] == 1.0f;
+  expect(once, c.name + ": every quantized activation, sum and scale once");
+  const jma::QactKOffsets o = jma::qact_k_offsets(c.batch, c.cols);
+  expect(o.classes >= (uint64_t)rows * c.cols * 2 && o.sums - o.classes >= (uint64_t)rows * c.cols * 2 &&
+             o.scales - o.sums >= (uint64_t)rows * KB * 32 && o.total - o.scales >= (uint64_t)rows * KB * 4,
+         c.name + ": activation scratch regions");
+  expect(o.total <= jma::qact_reserve_bytes((uint64_t)c.batch * c.cols), c.name + ": activation scratch");
 }
 
 // qmatvec_kernel / qkmatvec_kernel: the tile's weight units, the activation rows of each pass,
@@ -334,13 +344,19 @@ void walk(const Call& c) {
     total_rows += c.rows[i];
   }
   B.x = new float[(uint64_t)c.batch * c.cols];
-  B.aq = new int8_t[(uint64_t)c.batch * c.cols];
-  B.as = new float[(uint64_t)c.batch * K];
-  B.asum = new int[(uint64_t)c.batch * (c.cols / 16u)];
   B.written.assign(c.batch * total_rows, 0);
-  if (!kq && gemm_format(c.formats[0], c.batch)) {
+  if (gemm_format(c.formats[0], c.batch)) {
     const uint64_t rows32 = (uint64_t)jma::qact_tiles(c.batch) * 32u;
     B.act.assign(rows32 * c.cols, 0);
+    if (kq) {
+      B.act_class.assign(rows32 * c.cols, 0);
+      B.act_sum.assign(rows32 * K * 16u, 0);
+      B.act_scale_k.assign(rows32 * K, 0.0f);
+      walk_quant_k(c, B);
+    }
+  }
+  if (!kq && gemm_format(c.formats[0], c.batch)) {
+    const uint64_t rows32 = (uint64_t)jma::qact_tiles(c.batch) * 32u;
     B.act_scale.assign(rows32 * K, 0);
     walk_quant(c, B);
   }
@@ -356,9 +372,7 @@ void walk(const Call& c) {
   for (uint32_t fmt = 0; fmt <= 5; ++fmt) {
     if (std::find(c.formats.begin(), c.formats.end(), fmt) == c.formats.end()) continue;
     if (gemm_format(fmt, c.batch)) {
-      if (jma::qmat_kquant(fmt)) {
-        walk_gemm(c, fmt, B);
-      } else {
+      {
         // Every workgroup tile the planner may choose, the chosen one into the written counts.
         std::vector<uint32_t> fmt_rows;
         for (uint32_t i = 0; i < n; ++i)
@@ -367,7 +381,8 @@ void walk(const Call& c) {
         expect(chosen < jma::kQGemmShapes, c.name + ": product shape");
         for (uint32_t s = 0; s < jma::kQGemmShapes; ++s) {
           const std::vector<uint8_t> before = B.written;
-          walk_qgemm(c, fmt, jma::kQGemmShape[s], B);
+          if (jma::qmat_kquant(fmt)) walk_qkgemm(c, fmt, jma::qgemm_shape(fmt, s), B);
+          else walk_qgemm(c, fmt, jma::qgemm_shape(fmt, s), B);
           if (s != chosen) B.written = before;
         }
       }
@@ -391,9 +406,6 @@ void walk(const Call& c) {
     delete[] B.add[i];
   }
   delete[] B.x;
-  delete[] B.aq;
-  delete[] B.as;
-  delete[] B.asum;
 }
 
 }  // namespace
