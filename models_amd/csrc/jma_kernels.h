@@ -102,9 +102,14 @@ static_assert(sizeof(DecodeArgs) <= 4096, "DecodeArgs exceeds the kernel argumen
 
 struct PrefillArgs {
   KvView kv;
-  const float* q;       // [n][num_heads][dk], rotated
+  const float* q;       // [n][num_heads][dk], rotated, or raw with the factors below
   float* out;           // [n][num_heads][dv]
   int* err;
+  // Kernel 3 rotates raw queries itself (16-byte aligned): RoPE factors [max_positions][pairs], with
+  // split-half pairs over the whole head or interleaved ones in fours; null = q is as it will be used.
+  const float* cos_t;
+  const float* sin_t;
+  uint32_t pairs, neox;
   float qscale;         // score scale * log2(e)
   uint32_t n, start, seq, window;
   uint32_t num_heads, num_kv_heads, group;

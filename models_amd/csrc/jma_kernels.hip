@@ -186,8 +186,181 @@ __global__ __launch_bounds__(256) void rope_append_kernel(const AppendArgs a) {
   vb[kBlk] = (KV)v1;
 }
 
+// Kernel 1 for many consecutive rows (a prefill's): a workgroup takes the rows whose positions
+// share one 32-slot tile of the cache and one head of q, k or v, so that the norm sum of a head is
+// formed once (one thread a row, over the row staged in LDS, in order) instead of by each of its
+// threads, loads and stores are 16 bytes wide (8 for f16 keys), and a value tile is turned in LDS
+// and stored as whole 64-byte runs of positions instead of one element at a time. The arithmetic is
+// rope_append_kernel's. 2048 rows, 24 + 8 heads of 128, f16: 23.2 -> 14.0 us (5.4 TB/s of q, k and
+// v read, q and the cache written); with q and k norms, 1000 rows, 16 + 8 heads of 128, f32: 47 ->
+// 7.5 us; 1000 rows, 4 + 1 heads of 256, f16: 43.8 -> 5.5 us.
+// (kMaxD: the largest head length, which sizes the LDS.)
+template <typename KV, uint32_t kMaxD>
+__global__ __launch_bounds__(256) void append_tile_kernel(const AppendArgs a) {
+  constexpr bool kF16 = std::is_same<KV, _Float16>::value;
+  constexpr uint32_t kBlk = kF16 ? 32u : 16u;
+  __shared__ __attribute__((aligned(16))) float s_rows[32 * (kMaxD + 4)];  // [32][d + 4]
+  __shared__ float s_scale[32];
+  const uint32_t tid = threadIdx.x;
+  const uint32_t start = a.rows.start, first = (start / 32u + blockIdx.x) * 32u;  // the tile's first position
+  const uint32_t lo = max(start, first), hi = min(start + a.rows.count, first + 32u);
+  const uint32_t nr = hi - lo, row0 = lo - start;
+  const uint32_t tile = a.kv.ring ? first % a.kv.cap : first, in_tile = lo - first;  // slots
+  const uint32_t nq = a.q_out ? a.num_heads : 0u;
+  const uint32_t unit = blockIdx.y;
+  const bool is_v = unit >= nq + a.num_kv_heads, is_q = unit < nq;
+  const uint32_t h = is_q ? unit : is_v ? unit - nq - a.num_kv_heads : unit - nq;
+  const uint32_t heads = is_q ? a.num_heads : a.num_kv_heads, d = is_v ? a.dv : a.dk, d4 = d / 4u;
+  const uint32_t ld = d + 4u;  // floats of a staged row
+  const uint64_t stride = (uint64_t)heads * d;
+  const float* src = (is_q ? a.q : is_v ? a.v : a.k) + row0 * stride + (uint64_t)h * d;
+  const float* nw = is_q ? a.q_norm_w : a.k_norm_w;
+  const bool norm = is_v ? a.v_norm != 0u : nw != nullptr;
+
+  if (norm || is_v) {
+    for (uint32_t i = tid; i < nr * d4; i += 256u) {
+      const uint32_t r = i / d4, c = i % d4 * 4u;
+      *(float4_t*)(s_rows + r * ld + c) = *(const float4_t*)(src + r * stride + c);
+    }
+    __syncthreads();
+  }
+  if (norm) {
+    if (tid < nr) {
+#pragma clang fp contract(off)
+      const float* x = s_rows + tid * ld;
+      float ss = 0.0f;
+      for (uint32_t i = 0; i < d; i += 16u) {
+        float4_t v[4];
+#pragma unroll
+        for (int k = 0; k < 4; ++k) v[k] = *(const float4_t*)(x + i + 4 * k);
+#pragma unroll
+        for (int k = 0; k < 4; ++k)
+#pragma unroll
+          for (int e = 0; e < 4; ++e) ss = ss + v[k][e] * v[k][e];
+      }
+      const double rms = sqrt((double)(ss / (float)d + a.norm_eps));
+      s_scale[tid] = is_v ? (float)(1.0 / rms) : 1.0f / (float)rms;
+    }
+    __syncthreads();
+  }
+  if (is_v) {
+    KV* vb = (KV*)a.kv.v + a.rows.seq0 * a.kv.seq_stride_v + a.kv.layer_off_v + (uint64_t)h * a.kv.cap * d +
+             (uint64_t)(tile / kBlk) * d * kBlk;
+    auto value = [&](uint32_t r, uint32_t e) JMA_INL {  // row r of the launch's rows in this tile
+      const float x = s_rows[r * ld + e];
+      return norm ? x * s_scale[r] : x;
+    };
+    if (nr == 32u) {
+      // 16 bytes of positions a thread: f16 index 8 g .. 8 g + 7 of a column holds slots 4 g .. + 3
+      // and 16 + 4 g .. + 3 (perm32); f32 blocks of 16 slots hold them in order.
+      constexpr uint32_t kG = kF16 ? 4u : 8u;
+      for (uint32_t i = tid; i < d * kG; i += 256u) {
+        const uint32_t e = kF16 ? i / kG : i / 4u % d, g = kF16 ? i % kG : i % 4u + 4u * (i / (4u * d));
+        if constexpr (kF16) {
+          half8_t o;
+#pragma unroll
+          for (uint32_t k = 0; k < 8; ++k) o[k] = (KV)value(4u * g + k % 4u + 16u * (k / 4u), e);
+          *(half8_t*)(vb + e * kBlk + 8u * g) = o;
+        } else {
+          float4_t o;
+#pragma unroll
+          for (uint32_t k = 0; k < 4; ++k) o[k] = value(4u * g + k, e);
+          *(float4_t*)(vb + (uint64_t)(g / 4u) * d * kBlk + e * kBlk + 4u * (g % 4u)) = o;
+        }
+      }
+    } else {
+      for (uint32_t i = tid; i < nr * d; i += 256u) {
+        const uint32_t r = i % nr, e = i / nr, slot = in_tile + r;
+        const uint32_t at = kF16 ? perm32(slot) : slot % kBlk;
+        vb[(uint64_t)(slot / kBlk) * d * kBlk + e * kBlk + at] = (KV)value(r, e);
+      }
+    }
+    return;
+  }
+
+  KV* const kr = (KV*)a.kv.k + a.rows.seq0 * a.kv.seq_stride_k + a.kv.layer_off_k + (uint64_t)h * a.kv.cap * d;
+  // Four elements of row r at e, normalised; stored rotated.
+  auto load = [&](uint32_t r, uint32_t e) JMA_INL {
+#pragma clang fp contract(off)
+    if (!norm) return *(const float4_t*)(src + r * stride + e);
+    float4_t x = *(const float4_t*)(s_rows + r * ld + e);
+    const float4_t w = *(const float4_t*)(nw + e);
+    const float scale = s_scale[r];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) x[k] = x[k] * scale * w[k];
+    return x;
+  };
+  auto store = [&](uint32_t r, uint32_t e, float4_t x) JMA_INL {
+    if (is_q) {
+      *(float4_t*)(a.q_out + (row0 + r) * stride + (uint64_t)h * d + e) = x;
+    } else if constexpr (kF16) {
+      typedef _Float16 half4_t __attribute__((ext_vector_type(4)));
+      *(half4_t*)(kr + k_index(tile + in_tile + r, e, d, true)) =
+          half4_t{(KV)x[0], (KV)x[1], (KV)x[2], (KV)x[3]};
+    } else {
+      *(float4_t*)(kr + k_index(tile + in_tile + r, e, d, false)) = x;
+    }
+  };
+  // Work of a row: with split-half pairs, pairs / 4 chunks of both halves and the rest of the head;
+  // else chunks of four elements (two pairs).
+  const uint32_t pairs = a.cos_t ? a.pairs : 0u;
+  const uint32_t wide = a.neox ? pairs / 4u : 0u, chunks = d4 - wide;
+  for (uint32_t i = tid; i < nr * chunks; i += 256u) {
+    const uint32_t r = i / chunks, c = i % chunks;
+    const uint64_t at = (uint64_t)(lo + r) * a.pairs;
+    if (c < wide) {
+      float4_t x0 = load(r, 4u * c), x1 = load(r, pairs + 4u * c);
+      const float4_t cs = *(const float4_t*)(a.cos_t + at + 4u * c), sn = *(const float4_t*)(a.sin_t + at + 4u * c);
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        float y0 = x0[k], y1 = x1[k];
+        rotate_pair(y0, y1, cs[k], sn[k]);
+        x0[k] = y0, x1[k] = y1;
+      }
+      store(r, 4u * c, x0);
+      store(r, pairs + 4u * c, x1);
+      continue;
+    }
+    const uint32_t e = 4u * (c + wide);
+    float4_t x = load(r, e);
+    if (e < 2u * pairs && !a.neox) {
+      const float2_t cs = *(const float2_t*)(a.cos_t + at + e / 2u), sn = *(const float2_t*)(a.sin_t + at + e / 2u);
+#pragma unroll
+      for (int k = 0; k < 2; ++k) {
+        float y0 = x[2 * k], y1 = x[2 * k + 1];
+        rotate_pair(y0, y1, cs[k], sn[k]);
+        x[2 * k] = y0, x[2 * k + 1] = y1;
+      }
+    }
+    store(r, e, x);
+  }
+}
+
 hipError_t launch_append(const AppendArgs& a, bool f16, hipStream_t stream) {
   if (a.rows.count == 0) return hipSuccess;
+  // The tiled kernel's 16-byte accesses want aligned inputs, head lengths and rotary pairs in fours
+  // (the tables' rows start at multiples of the pairs); its LDS holds heads of up to 512.
+  const auto aligned = [](const void* p) { return ((uintptr_t)p & 15u) == 0; };
+  const uint32_t max_d = std::max(a.dk, a.dv), units = (a.q_out ? a.num_heads : 0u) + 2 * a.num_kv_heads;
+  // Without a norm to form, short launches are as fast or faster with a thread per pair (77 rows of
+  // 32 + 8 heads of 64: 11.5 against 12.3 us a prefill; 300 rows of keys and values 15.2 against 14.7).
+  const bool norms = a.q_norm_w || a.k_norm_w || a.v_norm;
+  const uint32_t min_rows = norms ? 8u : a.q_out ? 512u : 256u;
+  if (a.rows.contiguous && a.rows.count >= min_rows && a.pairs % 4 == 0 && a.dk % 16 == 0 && a.dv % 16 == 0 &&
+      max_d <= 512 && units <= 65535 && aligned(a.q) && aligned(a.k) && aligned(a.v) && aligned(a.q_out)) {
+    const uint32_t tiles = (a.rows.start + a.rows.count - 1) / 32 - a.rows.start / 32 + 1;
+    const dim3 grid(tiles, units), block(256);
+    if (f16) {
+      if (max_d <= 128) hipLaunchKernelGGL((append_tile_kernel<_Float16, 128>), grid, block, 0, stream, a);
+      else if (max_d <= 256) hipLaunchKernelGGL((append_tile_kernel<_Float16, 256>), grid, block, 0, stream, a);
+      else hipLaunchKernelGGL((append_tile_kernel<_Float16, 512>), grid, block, 0, stream, a);
+    } else {
+      if (max_d <= 128) hipLaunchKernelGGL((append_tile_kernel<float, 128>), grid, block, 0, stream, a);
+      else if (max_d <= 256) hipLaunchKernelGGL((append_tile_kernel<float, 256>), grid, block, 0, stream, a);
+      else hipLaunchKernelGGL((append_tile_kernel<float, 512>), grid, block, 0, stream, a);
+    }
+    return hipGetLastError();
+  }
   const dim3 grid(a.rows.count * a.blocks_per_row), block(256);
   if (f16) {
     hipLaunchKernelGGL(rope_append_kernel<_Float16>, grid, block, 0, stream, a);
@@ -1945,20 +2118,61 @@ __attribute__((amdgpu_waves_per_eu(D >= 256 ? 1 : 2))) void prefill_kernel(const
   // scale * log2(e) and rounded to f16. A scaled element beyond the f16 range (where the
   // reference's f32 scores stay finite) or infinite is reported like a non-finite score; a NaN
   // element makes its column's scores NaN, which the final normalisation reports.
+  // With a.cos_t the queries come raw and are rotated here, as the append kernel rotates keys (every
+  // product and sum rounded on its own): each lane holds whole pairs, both elements of an
+  // interleaved pair in one run of 8, both halves' elements of a split-half pair in runs kKS / 2
+  // apart (the whole head rotated). That saves writing and re-reading the rotated queries (C3: 50
+  // MB, 62.3 -> 56 us with the append).
   half8_t qf[kKS];
   {
     const float* qrow = a.q + ((uint64_t)crow * a.num_heads + head) * D + 8 * h;
     const float qs = col_ok ? a.qscale : 0.0f;
     float qmax = 0.0f;
-#pragma unroll
-    for (int ks = 0; ks < kKS; ++ks) {
-      const float4_t x0 = *(const float4_t*)(qrow + 16 * ks);
-      const float4_t x1 = *(const float4_t*)(qrow + 16 * ks + 4);
+    auto put = [&](int ks, const float4_t& x0, const float4_t& x1) JMA_INL {
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
         qmax = fmaxf(qmax, fmaxf(fabsf(x0[e] * qs), fabsf(x1[e] * qs)));
         qf[ks][e] = (_Float16)(x0[e] * qs);
         qf[ks][4 + e] = (_Float16)(x1[e] * qs);
+      }
+    };
+    auto rotate = [&](float4_t& x, float4_t& y, const float4_t& c, const float4_t& sn) JMA_INL {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        float u = x[e], v = y[e];
+        rotate_pair(u, v, c[e], sn[e]);
+        x[e] = u, y[e] = v;
+      }
+    };
+    if (a.cos_t == nullptr) {
+#pragma unroll
+      for (int ks = 0; ks < kKS; ++ks) put(ks, *(const float4_t*)(qrow + 16 * ks), *(const float4_t*)(qrow + 16 * ks + 4));
+    } else if (a.neox) {
+      const float* cr_ = a.cos_t + (uint64_t)cpos * (D / 2) + 8 * h;
+      const float* sr_ = a.sin_t + (uint64_t)cpos * (D / 2) + 8 * h;
+#pragma unroll
+      for (int ks = 0; ks < kKS / 2; ++ks) {
+        float4_t x0 = *(const float4_t*)(qrow + 16 * ks), x1 = *(const float4_t*)(qrow + 16 * ks + 4);
+        float4_t y0 = *(const float4_t*)(qrow + D / 2 + 16 * ks), y1 = *(const float4_t*)(qrow + D / 2 + 16 * ks + 4);
+        rotate(x0, y0, *(const float4_t*)(cr_ + 16 * ks), *(const float4_t*)(sr_ + 16 * ks));
+        rotate(x1, y1, *(const float4_t*)(cr_ + 16 * ks + 4), *(const float4_t*)(sr_ + 16 * ks + 4));
+        put(ks, x0, x1);
+        put(ks + kKS / 2, y0, y1);
+      }
+    } else {
+      const float* cr_ = a.cos_t + (uint64_t)cpos * a.pairs + 4 * h;
+      const float* sr_ = a.sin_t + (uint64_t)cpos * a.pairs + 4 * h;
+#pragma unroll
+      for (int ks = 0; ks < kKS; ++ks) {
+        float4_t x0 = *(const float4_t*)(qrow + 16 * ks), x1 = *(const float4_t*)(qrow + 16 * ks + 4);
+        if (16u * ks + 8u * h < 2u * a.pairs) {  // the rotary pairs come in fours
+          const float4_t c = *(const float4_t*)(cr_ + 8 * ks), sn = *(const float4_t*)(sr_ + 8 * ks);
+          float4_t u{x0[0], x0[2], x1[0], x1[2]}, v{x0[1], x0[3], x1[1], x1[3]};
+          rotate(u, v, c, sn);
+          x0 = float4_t{u[0], v[0], u[1], v[1]};
+          x1 = float4_t{u[2], v[2], u[3], v[3]};
+        }
+        put(ks, x0, x1);
       }
     }
     if (__ballot(col_ok && !(qmax < 65520.0f)) != 0 && lane == 0) atomicOr(a.err, 1);

@@ -371,11 +371,11 @@ void run_append(jmodels_attn_context* ctx, jmodels_attn_kv* kv, const LayerCall&
     a.pairs = lc.rope->pairs;
   }
   a.neox = lc.neox;
-  a.num_heads = lc.num_heads;
+  a.num_heads = q_out ? lc.num_heads : 0u;  // queries nobody reads are not rotated
   a.num_kv_heads = lc.hkv;
   a.dk = lc.dk;
   a.dv = lc.dv;
-  a.blocks_per_row = append_blocks_per_row(lc.num_heads, lc.hkv, lc.dk, lc.dv);
+  a.blocks_per_row = append_blocks_per_row(a.num_heads, lc.hkv, lc.dk, lc.dv);
   if (lc.norm) {
     a.q_norm_w = lc.norm->d_q;
     a.k_norm_w = lc.norm->d_k;
@@ -609,8 +609,10 @@ void check_prefill_shape(const jmodels_attn_kv* kv, const LayerCall& lc) {
 // Causal attention of rows start .. start+n-1 whose K/V are cached and whose rotated queries are
 // q (computeBatchedAttention, llama/LlamaForwardPass.java:1515-1541): row b attends
 // [first(start+b), start+b], on the kernel prefill_path picks.
+// raw: q is not rotated yet and the f16 MFMA prefill does it (prefill_rotates).
 void attend_causal_impl(jmodels_attn_context* ctx, const jmodels_attn_kv* kv, const LayerCall& lc,
-                        uint32_t sequence, uint32_t start, uint32_t n, const float* q, float* out) {
+                        uint32_t sequence, uint32_t start, uint32_t n, const float* q, float* out,
+                        bool raw = false) {
   const uint64_t qdim = (uint64_t)lc.num_heads * lc.dk;
   const uint64_t odim = (uint64_t)lc.num_heads * lc.dv;
   const PrefillPath path = prefill_path(kv, lc);
@@ -664,6 +666,12 @@ void attend_causal_impl(jmodels_attn_context* ctx, const jmodels_attn_kv* kv, co
     jma::PrefillArgs a{};
     a.kv = kv->view(lc.layer);
     a.q = q;
+    if (raw && lc.rope) {
+      a.cos_t = lc.rope->d_cos;
+      a.sin_t = lc.rope->d_sin;
+      a.pairs = lc.rope->pairs;
+      a.neox = lc.neox;
+    }
     a.qscale = lc.scale * 1.4426950408889634f;
     a.out = out;
     a.err = ctx->d_err;
@@ -720,22 +728,37 @@ void validate_causal(const jmodels_attn_kv* kv, const LayerCall& lc, uint32_t se
   else if (first < start) kv->require_range(sequence, lc.layer, first, start - 1);
 }
 
+// Whether the f16 MFMA prefill can take a call's queries as they come: no norm to apply (a head's
+// sum of squares in order is the append kernel's work), aligned for its 16-byte loads, and rotary
+// pairs that a lane holds whole.
+// Small prefills keep the rotated copy: the factors' loads lengthen the prologue of a launch that is
+// all latency (77 rows of 32 heads of 64: 12.3 against 11.7 us; 300 rows 14.7 against 15.8).
+constexpr uint64_t kRotateMinHeads = 8192;  // query rows x heads
+
+bool prefill_rotates(const jmodels_attn_kv* kv, const LayerCall& lc, uint32_t n, const float* q) {
+  if ((uint64_t)n * lc.num_heads < kRotateMinHeads) return false;
+  if (prefill_path(kv, lc) != PrefillPath::kF16 || (lc.norm && lc.norm->d_q) || ((uintptr_t)q & 15u) != 0) return false;
+  return !lc.rope || (lc.neox ? lc.rope->pairs * 2 == lc.dk : lc.rope->pairs % 4 == 0);
+}
+
 void prefill_impl(jmodels_attn_context* ctx, jmodels_attn_kv* kv, const LayerCall& lc,
                   uint32_t sequence, uint32_t start, uint32_t n, const float* q, const float* k,
                   const float* v, float* out) {
   const uint64_t qdim = (uint64_t)lc.num_heads * lc.dk;
   check_prefill_shape(kv, lc);
   validate_causal(kv, lc, sequence, start, n, false);
-  ctx->qrot.reserve((size_t)n * qdim * sizeof(float), ctx->stream, "prefill rotated queries");
+  const bool raw = prefill_rotates(kv, lc, n, q);
+  if (!raw) ctx->qrot.reserve((size_t)n * qdim * sizeof(float), ctx->stream, "prefill rotated queries");
+  float* const qrot = raw ? nullptr : (float*)ctx->qrot.ptr;
   // One launch appends every row: consecutive positions of one sequence need no row table.
   jma::RowList rows{};
   rows.count = n;
   rows.contiguous = 1;
   rows.seq0 = sequence;
   rows.start = start;
-  run_append(ctx, kv, lc, rows, q, k, v, (float*)ctx->qrot.ptr);
+  run_append(ctx, kv, lc, rows, q, k, v, qrot);
   for (uint32_t i = 0; i < n; ++i) kv->mark(sequence, lc.layer, start + i);
-  attend_causal_impl(ctx, kv, lc, sequence, start, n, (const float*)ctx->qrot.ptr, out);
+  attend_causal_impl(ctx, kv, lc, sequence, start, n, raw ? q : qrot, out, raw);
 }
 
 int32_t collect_errors(jmodels_attn_context* ctx) {
