@@ -65,7 +65,7 @@ struct DecodeArgs {
   const float* v_new;   // [count][num_kv_heads * dv]
   const float* cos_t;   // RoPE factors [max_positions][pairs]; null = no RoPE
   const float* sin_t;
-  int* err;             // bit 0: non-finite score seen
+  int* err;             // byte 0: non-finite score seen; byte 1: a reducer gave up waiting
   KvView kv;
   void* k_base;         // non-null: the rows are contiguous positions of one sequence, every row
   void* v_base;         // has the same split count, one head group; the layer's K / V base for

@@ -43,6 +43,13 @@ __device__ __forceinline__ uint32_t perm32(uint32_t r) {
   return 8u * ((r & 15u) >> 2) + 4u * (r >> 4) + (r & 3u);
 }
 
+// Raises an error in the context's error word, in host memory (one byte per kind: a plain store
+// from any number of waves, where an atomic would need the bus to carry it).
+constexpr int kErrNonFinite = 0, kErrTimeout = 1;
+__device__ __forceinline__ void report(int* err, int kind) {
+  __hip_atomic_store((uint8_t*)err + kind, (uint8_t)1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
 __device__ __forceinline__ uint32_t slot_of(const KvView& kv, uint32_t position) {
   return kv.ring ? position % kv.cap : position;
 }
@@ -761,7 +768,7 @@ __device__ __forceinline__ void reduce_group(float* part, uint64_t item0, uint32
       for (int c = 0; c < 4; ++c) X[c] += dpp<kDppHalfMirror>(X[c]);
     }
     if (qok && r == 0) {
-      if (!(L > 0.0f) && e == 0) atomicOr(err, 1);  // all -inf, or a NaN / +inf score
+      if (!(L > 0.0f) && e == 0) report(err, kErrNonFinite);  // all -inf, or a NaN / +inf score
       *(float4_t*)(out + hs * OS + e) = X * __builtin_amdgcn_rcpf(L);  // L >= 1: no denormals
     }
     // Clear-back of the acc words, after the output store.
@@ -773,7 +780,7 @@ __device__ __forceinline__ void reduce_group(float* part, uint64_t item0, uint32
     const uint32_t o = k / nreal, hs = k % nreal;
     clear_part(rs, base(o + (o >= split ? 1u : 0u), hs) + DV * 4);
   }
-  if (timed_out) atomicOr(err, 2);
+  if (timed_out) report(err, kErrTimeout);
 }
 
 // One workgroup = one work item (row, kv head, head group of <= 16 query heads, split); its
@@ -1479,7 +1486,7 @@ __global__ __launch_bounds__(64 * decode_waves(DK)) void decode_kernel(
     float4_t aw;
     wave_partial<DVS, kW>(s_acc, s_ml, hs, e, mx, lw, aw);
     if (ns == 1) {
-      if (!(lw > 0.0f) && e == 0) atomicOr(err, 1);  // all -inf, or a NaN / +inf score
+      if (!(lw > 0.0f) && e == 0) report(err, kErrNonFinite);  // all -inf, or a NaN / +inf score
       *(float4_t*)(o_grp + hs * DV + e) = aw * __builtin_amdgcn_rcpf(lw);
     } else if (!fused) {  // reduce_kernel combines the splits after this launch
       // Column slices write their columns into the head group's item; (m, l) are the same in
@@ -1650,7 +1657,7 @@ __global__ __launch_bounds__(64 * kWaves) void reduce_kernel(const float* p_acc,
     lt += s_l[i];
     xt += s_x[i][q];
   }
-  if (!(lt > 0.0f) && q == 0 && chunk == 0) atomicOr(a.err, 1);  // all -inf, NaN or +inf
+  if (!(lt > 0.0f) && q == 0 && chunk == 0) report(a.err, kErrNonFinite);  // all -inf, NaN or +inf
   if (e < DV) *(float4_t*)(out_p + ((uint64_t)row * p_heads + head) * DV + e) = xt * __builtin_amdgcn_rcpf(lt);
 }
 
@@ -1938,7 +1945,7 @@ __device__ __forceinline__ void split_exchange(const PrefillArgs& a, uint32_t pa
   const float e0 = m0 == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(m0 - M);
   const float e1 = m1 == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(m1 - M);
   const float L = fmaf(l1, e1, l0 * e0);
-  if (__ballot(col_ok && !(L > 0.0f && L < INFINITY)) != 0 && lane == 0) atomicOr(a.err, 1);
+  if (__ballot(col_ok && !(L > 0.0f && L < INFINITY)) != 0 && lane == 0) report(a.err, kErrNonFinite);
   const float inv = L > 0.0f ? 1.0f / L : 0.0f;
   float* const orow = a.out + ((uint64_t)crow * a.num_heads + head) * D + 4 * h;
 #pragma unroll
@@ -2175,7 +2182,7 @@ __attribute__((amdgpu_waves_per_eu(D >= 256 ? 1 : 2))) void prefill_kernel(const
         put(ks, x0, x1);
       }
     }
-    if (__ballot(col_ok && !(qmax < 65520.0f)) != 0 && lane == 0) atomicOr(a.err, 1);
+    if (__ballot(col_ok && !(qmax < 65520.0f)) != 0 && lane == 0) report(a.err, kErrNonFinite);
   }
 
   // Softmax state, set up by each pass: l accumulates in two chains (l, lb), summed at the end;
@@ -2511,7 +2518,7 @@ __attribute__((amdgpu_waves_per_eu(D >= 256 ? 1 : 2))) void prefill_kernel(const
   }
   if (!split) {
     const bool bad = col_ok && !(L > 0.0f && L < INFINITY);
-    if (__ballot(bad) != 0 && lane == 0) atomicOr(a.err, 1);
+    if (__ballot(bad) != 0 && lane == 0) report(a.err, kErrNonFinite);
     const float inv = L > 0.0f ? 1.0f / L : 0.0f;
 #pragma unroll
     for (int r = 0; r < Q; ++r) wr[r] *= inv;
@@ -2825,7 +2832,7 @@ __global__ __launch_bounds__(64 * W) void prefill_slice_kernel(const PrefillArgs
 
   const float L = half_sum(l + lb);
   const bool bad = col_ok && !(L > 0.0f && L < INFINITY);
-  if (__ballot(bad) != 0 && lane == 0) atomicOr(a.err, 1);
+  if (__ballot(bad) != 0 && lane == 0) report(a.err, kErrNonFinite);
   const float inv = L > 0.0f ? 1.0f / L : 0.0f;
   if (col_ok) {
     float* const orow = a.out + ((uint64_t)crow * a.num_heads + head) * D + 4 * h;
@@ -2998,7 +3005,7 @@ __global__ __launch_bounds__(256) void prefill_pair_kernel(const PrefillArgs a) 
         qf[i][4 + t] = (_Float16)(x1[t] * qs);
       }
     }
-    if (__ballot(col_ok && !(qmax < 65520.0f)) != 0 && lane == 0) atomicOr(a.err, 1);
+    if (__ballot(col_ok && !(qmax < 65520.0f)) != 0 && lane == 0) report(a.err, kErrNonFinite);
     // The q operands stay in the accumulation registers (matrix ops read them there), leaving
     // the vector registers to O^T, the scores and the tile operands.
 #pragma unroll
@@ -3172,7 +3179,7 @@ __global__ __launch_bounds__(256) void prefill_pair_kernel(const PrefillArgs a) 
 
   const float L = half_sum(l + lb);
   const bool bad = col_ok && !(L > 0.0f && L < INFINITY);
-  if (__ballot(bad) != 0 && lane == 0) atomicOr(a.err, 1);
+  if (__ballot(bad) != 0 && lane == 0) report(a.err, kErrNonFinite);
   const float inv = L > 0.0f ? 1.0f / L : 0.0f;
   if (col_ok) {
     float* const orow = a.out + ((uint64_t)crow * a.num_heads + head) * D + 4 * h;

@@ -148,7 +148,10 @@ int env_int(const char* name, int fallback) {
 struct jmodels_attn_context {
   int device = 0;
   hipStream_t stream = nullptr;
-  int* d_err = nullptr;
+  // Host memory the kernels reach: the error word, then room for the inputs and the output of a
+  // small host-buffer call, which its kernel reads and writes in place.
+  unsigned char* host = nullptr;
+  int* err = nullptr;
   DeviceBuffer part_acc, part_ml, part_f, counters, pf_part, pf_tickets, qrot, stage_q, stage_k, stage_v, stage_out;
   DeviceBuffer qact;                // Q8_0 activations of prefill-sized projections
   DeviceBuffer pp_part, pp_tickets; // split stripe pairs of the head-dim-512 f16 prefill
@@ -434,7 +437,7 @@ void run_attend_rows(jmodels_attn_context* ctx, const jmodels_attn_kv* kv, const
   a.kv = kv->view(lc.layer);
   a.q = q;
   a.out = out;
-  a.err = ctx->d_err;
+  a.err = ctx->err;
   a.qscale = lc.scale * 1.4426950408889634f;
   a.num_heads = lc.num_heads;
   a.group = lc.group;
@@ -622,7 +625,7 @@ void attend_causal_impl(jmodels_attn_context* ctx, const jmodels_attn_kv* kv, co
     a.q = q;
     a.qscale = lc.scale * 1.4426950408889634f;
     a.out = out;
-    a.err = ctx->d_err;
+    a.err = ctx->err;
     a.n = n;
     a.start = start;
     a.seq = sequence;
@@ -674,7 +677,7 @@ void attend_causal_impl(jmodels_attn_context* ctx, const jmodels_attn_kv* kv, co
     }
     a.qscale = lc.scale * 1.4426950408889634f;
     a.out = out;
-    a.err = ctx->d_err;
+    a.err = ctx->err;
     a.n = n;
     a.start = start;
     a.seq = sequence;
@@ -761,14 +764,12 @@ void prefill_impl(jmodels_attn_context* ctx, jmodels_attn_kv* kv, const LayerCal
   attend_causal_impl(ctx, kv, lc, sequence, start, n, raw ? q : qrot, out, raw);
 }
 
-int32_t collect_errors(jmodels_attn_context* ctx) {
-  hip_check(hipStreamSynchronize(ctx->stream), "hipStreamSynchronize");
-  int err = 0;
-  hip_check(hipMemcpy(&err, ctx->d_err, sizeof(int), hipMemcpyDeviceToHost), "read error word");
+// The stream has been waited for: raises what its kernels reported since the last time.
+void raise_errors(jmodels_attn_context* ctx) {
+  const int err = *(volatile int*)ctx->err;
   if (err != 0) {
-    int zero = 0;
-    hip_check(hipMemcpy(ctx->d_err, &zero, sizeof(int), hipMemcpyHostToDevice), "reset error word");
-    if (err & 2) {
+    *(volatile int*)ctx->err = 0;
+    if (err & 0xFF00) {
       // A reducer gave up waiting: tickets and partial words may be left set; clear them.
       for (DeviceBuffer* b : {&ctx->part_f})
         if (b->ptr) hip_check(hipMemset(b->ptr, 0xFF, b->bytes), "reset partials");
@@ -779,7 +780,11 @@ int32_t collect_errors(jmodels_attn_context* ctx) {
     }
     fail(JMODELS_ATTN_NON_FINITE, "softmax input contains NaN or positive infinity");
   }
-  return JMODELS_ATTN_OK;
+}
+
+void collect_errors(jmodels_attn_context* ctx) {
+  hip_check(hipStreamSynchronize(ctx->stream), "hipStreamSynchronize");
+  raise_errors(ctx);
 }
 
 void set_device(const jmodels_attn_context* ctx) { hip_check(hipSetDevice(ctx->device), "hipSetDevice"); }
@@ -792,6 +797,43 @@ T* stage(DeviceBuffer& buf, const T* host, uint64_t elems, hipStream_t stream) {
               "copy to device");
   return (T*)buf.ptr;
 }
+
+// A small host-buffer call's inputs and output in the context's host memory: the kernel reads and
+// writes them over the bus, which takes less than a copy each way (one layer-step of 16 + 8 heads of
+// 128 at 512 positions: 63 us with three copies in, one out and one of the error word; see the
+// sizes below for where the copies are better again).
+constexpr size_t kHostErr = 256, kHostIn = 64 << 10, kHostOut = 64 << 10;
+constexpr size_t kHostBytes = kHostErr + kHostIn + kHostOut;
+
+class HostCall {
+ public:
+  HostCall(jmodels_attn_context* ctx, uint64_t in_elems, uint64_t out_elems)
+      : ctx_(ctx), fits_(in_elems * sizeof(float) + 3 * 256 <= kHostIn &&
+                         out_elems * sizeof(float) <= kHostOut) {}
+  ~HostCall() {
+    // A launch failed after another was sent: the next call may not overwrite what that one reads.
+    if (used_ != 0) (void)hipStreamSynchronize(ctx_->stream);
+  }
+  explicit operator bool() const { return fits_; }
+  const float* put(const float* x, uint64_t elems) {
+    float* at = (float*)(ctx_->host + kHostErr) + used_;
+    memcpy(at, x, elems * sizeof(float));
+    used_ += round_up(elems, 64);
+    return at;
+  }
+  float* out() const { return (float*)(ctx_->host + kHostErr + kHostIn); }
+  void finish(float* dst, uint64_t elems) {
+    hip_check(hipStreamSynchronize(ctx_->stream), "hipStreamSynchronize");
+    used_ = 0;
+    memcpy(dst, out(), elems * sizeof(float));
+    raise_errors(ctx_);
+  }
+
+ private:
+  jmodels_attn_context* ctx_;
+  bool fits_;
+  uint64_t used_ = 0;
+};
 
 // One matrix of a quantized projection call.
 struct QuantMatrix {
@@ -982,14 +1024,15 @@ jmodels_attn_context* jmodels_attn_context_create(int32_t device) {
     ctx->unfused = env_int("JMA_UNFUSED", 0) != 0;
     try {
       hip_check(hipStreamCreateWithFlags(&ctx->stream, hipStreamNonBlocking), "hipStreamCreate");
-      hip_check(hipMalloc(&ctx->d_err, sizeof(int)), "hipMalloc error word");
-      hip_check(hipMemset(ctx->d_err, 0, sizeof(int)), "hipMemset error word");
+      hip_check(hipHostMalloc((void**)&ctx->host, kHostBytes, hipHostMallocCoherent), "hipHostMalloc");
+      ctx->err = (int*)ctx->host;
+      *ctx->err = 0;
       // The device's fixed scratch: its address, and its exchange regions prepared, once per
       // device (the allocation-free entry point then allocates nothing).
       hip_check(jma::fixed_scratch(device, ctx->stream, &ctx->fixed), "fixed scratch");
     } catch (...) {
       if (ctx->stream) (void)hipStreamDestroy(ctx->stream);
-      if (ctx->d_err) (void)hipFree(ctx->d_err);
+      if (ctx->host) (void)hipHostFree(ctx->host);
       delete ctx;
       throw;
     }
@@ -1007,7 +1050,7 @@ int32_t jmodels_attn_context_destroy(jmodels_attn_context* ctx) {
                             &ctx->stage_k, &ctx->stage_v, &ctx->stage_out, &ctx->qact, &ctx->pp_part,
                             &ctx->pp_tickets})
       b->release();
-    (void)hipFree(ctx->d_err);
+    (void)hipHostFree(ctx->host);
     (void)hipStreamDestroy(ctx->stream);
     delete ctx;
   });
@@ -1490,6 +1533,11 @@ static int32_t attend_entry(bool device, jmodels_attn_context* ctx, const jmodel
       run_attend(ctx, kv, lc, count, sequences, positions, q, out);
       return;
     }
+    HostCall hc(ctx, qn, on);
+    if (hc) {
+      run_attend(ctx, kv, lc, count, sequences, positions, hc.put(q, qn), hc.out());
+      return hc.finish(out, on);
+    }
     const float* dq = stage(ctx->stage_q, q, qn, ctx->stream);
     float* dout = stage<float>(ctx->stage_out, nullptr, on, ctx->stream);
     run_attend(ctx, kv, lc, count, sequences, positions, dq, dout);
@@ -1554,7 +1602,13 @@ static int32_t decode_entry(bool device, jmodels_attn_context* ctx, jmodels_attn
     const float* dk = k;
     const float* dv = v;
     float* dout = out;
-    if (!device) {
+    HostCall hc(ctx, qn + kn + vn, on);
+    if (!device && hc) {
+      dq = hc.put(q, qn);
+      dk = hc.put(k, kn);
+      dv = hc.put(v, vn);
+      dout = hc.out();
+    } else if (!device) {
       dq = stage(ctx->stage_q, q, qn, ctx->stream);
       dk = stage(ctx->stage_k, k, kn, ctx->stream);
       dv = stage(ctx->stage_v, v, vn, ctx->stream);
@@ -1586,6 +1640,7 @@ static int32_t decode_entry(bool device, jmodels_attn_context* ctx, jmodels_attn
       run_attend(ctx, kv, lc, count, sequences, positions, qrot, dout, fixed);
     }
     if (device) return;
+    if (hc) return hc.finish(out, on);
     hip_check(hipMemcpyAsync(out, dout, on * sizeof(float), hipMemcpyDeviceToHost, ctx->stream),
               "copy out");
     collect_errors(ctx);

@@ -48,6 +48,9 @@ typedef struct hipDeviceProp_t {
 extern "C" {
 hipError_t hipMalloc(void** ptr, size_t size);
 hipError_t hipFree(void* ptr);
+constexpr unsigned int hipHostMallocCoherent = 0x40000000u;
+hipError_t hipHostMalloc(void** ptr, size_t size, unsigned int flags);
+hipError_t hipHostFree(void* ptr);
 hipError_t hipMemcpy(void* dst, const void* src, size_t bytes, hipMemcpyKind kind);
 hipError_t hipMemcpyAsync(void* dst, const void* src, size_t bytes, hipMemcpyKind kind, hipStream_t stream);
 hipError_t hipMemset(void* dst, int value, size_t bytes);

@@ -169,6 +169,11 @@ hipError_t hipMemcpyAsync(void* dst, const void* src, size_t bytes, hipMemcpyKin
   return hipSuccess;
 }
 
+// Host memory the device reaches: a live allocation like the others.
+hipError_t hipHostMalloc(void** ptr, size_t size, unsigned int) { return hipMalloc(ptr, size); }
+
+hipError_t hipHostFree(void* ptr) { return hipFree(ptr); }
+
 hipError_t hipMemset(void* dst, int value, size_t bytes) {
   Op op{Op::kSet};
   op.dst = dst;
