@@ -341,10 +341,13 @@ __global__ __launch_bounds__(64 * NB * NW, 2) void qkgemm_kernel(
   constexpr uint32_t kPPW = (kPieces + kWaves - 1) / kWaves;
   constexpr uint32_t kScales = (kB + 63) / 64;  // 64-row pieces of activation scales
   static_assert(kUnits <= kThreads, "at most one staged half block per thread");
-  // A wave's loads in step g of a block.
+  // A wave's loads in step g of a block. The barrier that closes a step leaves that step's and the one
+  // before's in flight, so what a step loads is there three steps later: step 4's scales in step 7.
+  constexpr int kScaleStep = 4;
+  static_assert(kScaleStep + 3 <= 7, "the last step reads the block's activation scales");
   constexpr auto loads = [](int g) {
     return (int)kPPW + (g % 2 == 0 ? 2 : 0) + (g == 3 ? (FMT == 4 ? 3 : 1) : 0) + (g == 4 ? BT : 0) +
-           (g == 5 ? (int)kScales : 0);
+           (g == kScaleStep ? (int)kScales : 0);
   };
   __shared__ __attribute__((aligned(16))) _Float16 w0[kW * 32], w1[kW * 32];
   __shared__ __attribute__((aligned(16))) _Float16 a0[kB * 32], a1[kB * 32], a2[kB * 32], a3[kB * 32];
@@ -476,7 +479,7 @@ __global__ __launch_bounds__(64 * NB * NW, 2) void qkgemm_kernel(
 #pragma unroll
       for (int i = 0; i < BT; ++i) sum_op[i] = *(const half8_t*)(sums_at[i] + (uint64_t)kb * 512u);
     }
-    if constexpr (g == 5) {
+    if constexpr (g == kScaleStep) {
 #pragma unroll
       for (uint32_t i = 0; i < kScales; ++i) dma4(scales, s_as + 64 * i, scale_off[i], kb * 128u);
     }
