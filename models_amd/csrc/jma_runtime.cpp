@@ -772,9 +772,9 @@ void raise_errors(jmodels_attn_context* ctx) {
     if (err & 0xFF00) {
       // A reducer gave up waiting: tickets and partial words may be left set; clear them.
       for (DeviceBuffer* b : {&ctx->part_f})
-        if (b->ptr) hip_check(hipMemset(b->ptr, 0xFF, b->bytes), "reset partials");
+        if (b->ptr) hip_check(hipMemsetAsync(b->ptr, 0xFF, b->bytes, ctx->stream), "reset partials");
       for (DeviceBuffer* b : {&ctx->counters, &ctx->pf_tickets, &ctx->pp_tickets})
-        if (b->ptr) hip_check(hipMemset(b->ptr, 0, b->bytes), "reset tickets");
+        if (b->ptr) hip_check(hipMemsetAsync(b->ptr, 0, b->bytes, ctx->stream), "reset tickets");
       hip_check(jma::fixed_scratch_reset(ctx->fixed, ctx->stream), "reset fixed scratch");
       fail(JMODELS_ATTN_DEVICE_ERROR, "cross-split reduction timed out waiting for a partial");
     }

@@ -96,7 +96,10 @@ class DeviceArray:
         return out
 
     def zero(self) -> None:
+        # hipMemset may return before the device has written, and a context's non-blocking stream
+        # does not wait for the null stream.
         check(hip().hipMemset(self.ptr, 0, self.nbytes), "hipMemset")
+        check(hip().hipStreamSynchronize(None), "hipStreamSynchronize")
 
     def at(self, offset_elems: int) -> int:
         """Device address of element ``offset_elems``."""
