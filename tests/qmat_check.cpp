@@ -3,10 +3,9 @@
 //
 // For each call below it routes every weight format the way quantized_matmul_impl does and plans
 // its launch with the runtime's own planner (jma_plan.h): prefill-sized batches run the
-// register-tiled product (qgemm_kernel, qkgemm_kernel, q6gemm_kernel) in tiles of kQGemmTile rows
-// x kQGemmTile activation rows over activations quantized once into scratch; the others run the
-// matrix-vector kernels (plan_qmat, qmat_group_rows), whose workgroups take `chunk` activation
-// rows per pass. It then walks every workgroup (x, y) of every launch the way the kernels index
+// matrix-core product (qgemm_kernel, qkgemm_kernel, q6gemm_kernel) in the workgroup tiles that
+// plan_qgemm picks, over activations quantized once into scratch; the others run the matrix-vector
+// kernels (plan_qmat, qmat_group_rows), whose workgroups take `chunk` activation rows per pass. It then walks every workgroup (x, y) of every launch the way the kernels index
 // memory: the matrix a workgroup serves (the last with tile0 <= x), its weight blocks, the
 // activations (or the quantized activation scratch) it reads, its LDS arrays, and every output,
 // bias and residual element it reads or writes. Every access touches an exactly sized heap array,

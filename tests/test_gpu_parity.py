@@ -997,6 +997,98 @@ def test_attend_causal_equals_prefill(hip):
         rope.close()
 
 
+PREFILL_TILE_CASES = {
+    # name: (f16 cache, heads, KV heads, d, rotary dim, NeoX pairs, norms, first position, rows). f16
+    # calls of 8192 (row, head) queries and more without a norm rotate q in the prefill kernel.
+    "rotated-in-kernel": (True, 12, 4, 128, 128, True, False, 0, 1001),
+    "rotated-in-kernel-interleaved-chunk": (True, 12, 4, 64, 64, False, False, 45, 701),
+    "rotated-in-kernel-partial": (True, 16, 2, 256, 128, False, False, 31, 513),
+    "at-the-rule": (True, 32, 8, 64, 64, True, False, 0, 256),
+    "below-the-rule": (True, 32, 8, 64, 64, True, False, 0, 255),
+    "neox-partial": (True, 32, 8, 128, 64, True, False, 1, 600),
+    "normed": (True, 4, 1, 256, 256, True, True, 33, 300),
+    "normed-8-rows": (True, 4, 1, 128, 128, True, True, 30, 8),
+    "normed-d512": (True, 8, 1, 512, 128, True, True, 0, 97),
+    "f32": (False, 16, 8, 128, 128, True, False, 17, 520),
+    "f32-normed": (False, 16, 8, 64, 64, False, True, 0, 65),
+}
+
+
+@pytest.mark.parametrize("case", list(PREFILL_TILE_CASES))
+def test_prefill_by_cache_tiles_equals_rows(hip, case):
+    """A prefill's append by 32-slot cache tiles (and queries rotated inside the f16 prefill) against
+    the row kernel and attend_causal on its rotated queries: the same arithmetic in the same order, so
+    the caches and the outputs agree bit for bit, ragged first and last tiles included; stored keys
+    are the oracle's bits where no norm goes before the rotation."""
+    half, hq, hkv, d, rd, neox, norms, start, n = PREFILL_TILE_CASES[case]
+    theta, total = 1e6, start + n
+    q = normal(21, f"pt/{case}/q", (total, hq * d))
+    k = normal(21, f"pt/{case}/k", (total, hkv * d))
+    v = normal(21, f"pt/{case}/v", (total, hkv * d))
+    rope = hip.rotary_table(rd, theta, 1.0, max_positions=total)
+    norm = hip.qk_norm(d, normal(21, f"pt/{case}/wq", (d,)) * 0.2 + 1.0,
+                       normal(21, f"pt/{case}/wk", (d,)) * 0.2 + 1.0, 1e-6) if norms else None
+    a = hip.kv_cache(1, total, hkv, d, d, half_precision=half)
+    b = hip.kv_cache(1, total, hkv, d, d, half_precision=half)
+    try:
+        layer = A.AttentionLayer(0, hq, neox=neox, rope=rope, qk_norm=norm)
+        if start:
+            a.append(layer, np.arange(start), q[:start], k[:start], v[:start])
+        got = a.prefill(layer, start, q[start:], k[start:], v[start:])
+        # Rows in reverse order: a list of positions, never a run of them.
+        order = np.arange(total)[::-1]
+        q_rot = b.append(layer, order, q[order], k[order], v[order]).reshape(total, -1)[::-1]
+        want = b.attend_causal(layer, start, np.ascontiguousarray(q_rot[start:]))
+        for x, y in zip(a.read(0, 0, total), b.read(0, 0, total)):
+            np.testing.assert_array_equal(x, y)
+        np.testing.assert_array_equal(got, want)
+        if not norms:
+            ref = rope_rows(k, range(total), hkv, d, rd, theta, neox)
+            keys = a.read(0, 0, total)[0].reshape(total, -1)
+            np.testing.assert_array_equal(keys, oracle.f16_round(ref) if half else ref)
+    finally:
+        a.close()
+        b.close()
+        rope.close()
+        if norm is not None:
+            norm.close()
+
+
+@pytest.mark.parametrize("sessions", [1, 21, 22])
+def test_host_decode_around_the_pinned_size(hip, sessions):
+    """Host-buffer decode of 12 x 64 inputs a row: 21 rows are the most that go through the context's
+    pinned memory (64 KiB of inputs with their alignment), 22 are copied. A NaN reported by one call
+    is raised by that call and is gone for the next."""
+    hq, hkv, d, prior, theta = 8, 2, 64, 40, 1e6
+    scale = A.default_scale(d)
+    rope = hip.rotary_table(d, theta, 1.0, max_positions=64)
+    kv = hip.kv_cache(1, 64, hkv, d, d, half_precision=False, sequences=sessions)
+    layer = A.AttentionLayer(0, hq, neox=True, rope=rope)
+    q, k, v = (normal(22, f"hp/{x}", (sessions, prior + 1, h * d))
+               for x, h in (("q", hq), ("k", hkv), ("v", hkv)))
+    seqs, last = np.arange(sessions), np.full(sessions, prior)
+    try:
+        for s in range(sessions):
+            kv.append(layer, np.arange(prior), q[s, :prior], k[s, :prior], v[s, :prior],
+                      sequences=np.full(prior, s))
+        bad = q[:, prior].copy()
+        bad[-1, 3] = np.nan
+        with pytest.raises(A.AttentionStatusError):
+            kv.decode(layer, last, bad, k[:, prior], v[:, prior], sequences=seqs)
+        got = kv.decode(layer, last, q[:, prior], k[:, prior], v[:, prior], sequences=seqs)
+        got = np.asarray(got).reshape(sessions, -1)
+        for s in range(sessions):
+            ref = OracleKv(1, 64, hkv * d, hkv * d)
+            ref.prefill_layer(0, 0, q[s, :prior], k[s, :prior], v[s, :prior], hq, hkv, d, d, theta,
+                              1.0, True, scale)
+            want, _, _ = ref.decode_layer(0, prior, q[s, prior], k[s, prior], v[s, prior], hq, hkv,
+                                          d, d, theta, 1.0, True, scale)
+            assert_f32_close(got[s], want, f"session {s} of {sessions}", head_dim=d)
+    finally:
+        kv.close()
+        rope.close()
+
+
 @pytest.mark.parametrize("d", [64, 256])
 @pytest.mark.parametrize("neox", [False, True])
 def test_split_plans_and_fusion_agree(hip, monkeypatch, neox, d):

@@ -107,7 +107,7 @@ def test_random_shapes_bit_exact(hip, fmt, batch, rows, cols):
 def test_kquant_random_shapes_bit_exact(hip, fmt, batch, rows, cols):
     """Q4_K, Q5_K and Q6_K with Q8_K activations: the device repeats backend-native's scalar row
     kernels' float order (the integer parts are exact in any order), so the outputs are the
-    oracle's bits; batches of 16 rows and more run as the register-tiled product (ragged tile
+    oracle's bits; batches of 16 rows and more run as the matrix-core product (ragged tile
     edges in both dimensions included), smaller ones in the matrix-vector kernel."""
     w = _kquant_weights(fmt, rows, cols, f"kq/{fmt}/{rows}/{cols}")
     x = synth.normal(11, f"kq/x/{batch}/{cols}", (batch, cols)) * 1.5
@@ -121,7 +121,7 @@ def test_q6_k_extreme_quants_and_scales(hip, batch):
     """Q6_K at the ends of its ranges: quants 0 and 63 (-32 and 31 after the offset), sub-block
     scales -128 and 127, activations quantized to +-127, and d = 1; the product stages
     scale x quant as 16 bits, and every output must still be the oracle's bits (matrix-vector
-    kernel at batch 5, register-tiled product at 32)."""
+    kernel at batch 5, matrix-core product at 32)."""
     rows, cols = 70, 512
     raw = np.zeros((rows, cols // 256, 210), np.uint8)
     for r in range(rows):
@@ -277,10 +277,46 @@ def test_prefill_sized_grouped_projection_with_addends(hip, mode):
             d.free()
 
 
+MATRIX_PRODUCT_EDGES = [
+    # (activation rows, weight rows, 256-element blocks of inputs): each workgroup tile of the
+    # product one short of, at and past its edges, and the fewest inputs it takes.
+    (16, 1, 1), (31, 127, 2), (32, 128, 1), (33, 129, 1),      # 32 x 128 tiles, then 64 x 64
+    (63, 63, 3), (65, 65, 2),
+    (1281, 1537, 1), (1279, 1535, 2),                          # 128 x 128 (Q5_K and Q6_K 128 x 64)
+]
+
+
+@pytest.mark.parametrize("fmt", [A.WEIGHTS_Q4_0, A.WEIGHTS_Q8_0, A.WEIGHTS_Q5_0, A.WEIGHTS_Q4_K,
+                                 A.WEIGHTS_Q5_K, A.WEIGHTS_Q6_K])
+@pytest.mark.parametrize("batch,rows,blocks", MATRIX_PRODUCT_EDGES)
+def test_matrix_product_tile_edges_bit_exact(hip, fmt, batch, rows, blocks):
+    """The f16 matrix-core product at the edges of its tiles, with a residual updated in place. The
+    activation rows run from 1e-5 to 10 in magnitude, so Q8_0 scales and scale products are subnormal
+    in 16 bits at one end; bit-exact, since every matrix-op sum is an integer below 2^24 or one exact
+    product."""
+    small = fmt in (A.WEIGHTS_Q4_0, A.WEIGHTS_Q8_0, A.WEIGHTS_Q5_0)
+    cols = 256 * blocks - (96 if small else 0)
+    w = (_weights if small else _kquant_weights)(fmt, rows, cols, f"edge/{fmt}/{rows}/{cols}")
+    x = synth.normal(11, f"edge/x/{batch}/{cols}", (batch, cols))
+    x = (x * np.logspace(-5, 1, batch)[:, None]).astype(np.float32)
+    resid = synth.normal(11, f"edge/r/{batch}/{rows}", (batch, rows)).astype(np.float32)
+    dw, dx, dout = (rt.DeviceArray.from_host(a) for a in (w, x, resid))
+    try:
+        hip.quantized_matmul_device(fmt, dw.ptr, w.size, dx.ptr, x.size, dout.ptr, resid.size, batch,
+                                    rows, cols, dout.ptr, A.ADDEND_RESIDUAL)
+        hip.synchronize()
+        got = dout.download().reshape(batch, rows)
+    finally:
+        for d in (dw, dx, dout):
+            d.free()
+    want = (oracle.quantized_matmul(fmt, w, x, batch, rows, cols) + resid).astype(np.float32)
+    _exact(got, want.reshape(batch, rows), f"fmt {fmt} {batch}x{rows}x{cols}")
+
+
 @pytest.mark.parametrize("case", ["q5_0-q8_0-q4_0 bias x300", "q8_0 wo residual x64",
                                   "q4_k-q5_k-q6_k residual x40", "q4_0 graph x96"])
 def test_prefill_sized_projections(hip, case):
-    """Prefill-sized batches in one launch per format (the register-tiled product on activations
+    """Prefill-sized batches in one launch per format (the matrix-core product on activations
     quantized once). Grouped calls with biases or residuals (in place for the output projection),
     mixed 32-element formats, a K-quant mix with Q6_K, and a captured graph replayed three times;
     every output bit-exact against the oracle."""
