@@ -996,7 +996,7 @@ def main() -> int:
                         "Q4_0 / Q8_0 / Q5_0 / Q4_K / Q5_K / Q6_K weights, activations quantized "
                         "(Q8_0 or Q8_K) in the launch (us, GB/s of weights); qkv_prefill2048_*: "
                         "C3's grouped Q/K/V (3072 -> 3072 + 1024 + 1024) over its 2048-row prompt, "
-                        "activations quantized once, then the register-tiled product (us, integer "
+                        "activations quantized once, then the matrix-core product (us, integer "
                         "TOPS); q4_k_m: Q and K in Q4_K, V in Q6_K",
             **proj,
         }
