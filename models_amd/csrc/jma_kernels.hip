@@ -200,7 +200,7 @@ __global__ __launch_bounds__(256) void rope_append_kernel(const AppendArgs a) {
 // and stored as whole 64-byte runs of positions instead of one element at a time. The arithmetic is
 // rope_append_kernel's. 2048 rows, 24 + 8 heads of 128, f16: 23.2 -> 14.0 us (5.4 TB/s of q, k and
 // v read, q and the cache written); with q and k norms, 1000 rows, 16 + 8 heads of 128, f32: 47 ->
-// 7.5 us; 1000 rows, 4 + 1 heads of 256, f16: 43.8 -> 5.5 us.
+// 7.5 us; 1000 rows, 4 + 1 heads of 256, f16: 43.8 -> 11.2 us (traced).
 // (kMaxD: the largest head length, which sizes the LDS.)
 template <typename KV, uint32_t kMaxD>
 __global__ __launch_bounds__(256) void append_tile_kernel(const AppendArgs a) {
@@ -1976,7 +1976,7 @@ __device__ __forceinline__ void split_exchange(const PrefillArgs& a, uint32_t pa
 // so the result is the softmax of the reference up to f16 rounding of q, k, v and p.
 // Up to D = 128 the kernel fits 256 registers per lane (two waves per SIMD), which also keeps
 // the matrix-op results in ordinary vector registers (no accumulation-register copies per tile).
-template <int D>
+template <int D, bool kRaw>
 __global__ __launch_bounds__(64 * pf::Shape<D>::S * pf::Shape<D>::Q)
 __attribute__((amdgpu_waves_per_eu(D >= 256 ? 1 : 2))) void prefill_kernel(const PrefillArgs a) {
   using namespace pf;
@@ -2125,7 +2125,7 @@ __attribute__((amdgpu_waves_per_eu(D >= 256 ? 1 : 2))) void prefill_kernel(const
   // scale * log2(e) and rounded to f16. A scaled element beyond the f16 range (where the
   // reference's f32 scores stay finite) or infinite is reported like a non-finite score; a NaN
   // element makes its column's scores NaN, which the final normalisation reports.
-  // With a.cos_t the queries come raw and are rotated here, as the append kernel rotates keys (every
+  // With kRaw (a.cos_t given) the queries come raw and are rotated here, as the append kernel rotates keys (every
   // product and sum rounded on its own): each lane holds whole pairs, both elements of an
   // interleaved pair in one run of 8, both halves' elements of a split-half pair in runs kKS / 2
   // apart (the whole head rotated). That saves writing and re-reading the rotated queries (C3: 50
@@ -2138,9 +2138,13 @@ __attribute__((amdgpu_waves_per_eu(D >= 256 ? 1 : 2))) void prefill_kernel(const
     auto put = [&](int ks, const float4_t& x0, const float4_t& x1) JMA_INL {
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
-        qmax = fmaxf(qmax, fmaxf(fabsf(x0[e] * qs), fabsf(x1[e] * qs)));
-        qf[ks][e] = (_Float16)(x0[e] * qs);
-        qf[ks][4 + e] = (_Float16)(x1[e] * qs);
+        // Rounded to f32 first, always: the compiler would fold some of these products into the
+        // conversion, others in another instance, and the two forms' last bits differ.
+        float p0 = x0[e] * qs, p1 = x1[e] * qs;
+        asm("" : "+v"(p0), "+v"(p1));
+        qmax = fmaxf(qmax, fmaxf(fabsf(p0), fabsf(p1)));
+        qf[ks][e] = (_Float16)p0;
+        qf[ks][4 + e] = (_Float16)p1;
       }
     };
     auto rotate = [&](float4_t& x, float4_t& y, const float4_t& c, const float4_t& sn) JMA_INL {
@@ -2151,7 +2155,7 @@ __attribute__((amdgpu_waves_per_eu(D >= 256 ? 1 : 2))) void prefill_kernel(const
         x[e] = u, y[e] = v;
       }
     };
-    if (a.cos_t == nullptr) {
+    if constexpr (!kRaw) {
 #pragma unroll
       for (int ks = 0; ks < kKS; ++ks) put(ks, *(const float4_t*)(qrow + 16 * ks), *(const float4_t*)(qrow + 16 * ks + 4));
     } else if (a.neox) {
@@ -3200,7 +3204,11 @@ hipError_t launch_prefill_t(PrefillArgs a, hipStream_t stream) {
   if (blocks > 0x7fffffffu || a.split_blocks > a.row_blocks) return hipErrorInvalidValue;
   if ((uint64_t)a.kv.cap * D * 2 > 0x7fffffffu) return hipErrorInvalidValue;  // 32-bit tile offsets
   if (a.split_blocks > 0 && (a.part == nullptr || a.tickets == nullptr)) return hipErrorInvalidValue;
-  hipLaunchKernelGGL((prefill_kernel<D>), dim3((uint32_t)blocks), dim3(64 * S * Q), 0, stream, a);
+  // Instances of their own: the rotation's code and registers would lengthen launches without it.
+  if (a.cos_t)
+    hipLaunchKernelGGL((prefill_kernel<D, true>), dim3((uint32_t)blocks), dim3(64 * S * Q), 0, stream, a);
+  else
+    hipLaunchKernelGGL((prefill_kernel<D, false>), dim3((uint32_t)blocks), dim3(64 * S * Q), 0, stream, a);
   return hipGetLastError();
 }
 
