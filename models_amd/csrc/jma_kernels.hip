@@ -200,7 +200,7 @@ __global__ __launch_bounds__(256) void rope_append_kernel(const AppendArgs a) {
 // and stored as whole 64-byte runs of positions instead of one element at a time. The arithmetic is
 // rope_append_kernel's. 2048 rows, 24 + 8 heads of 128, f16: 23.2 -> 14.0 us (5.4 TB/s of q, k and
 // v read, q and the cache written); with q and k norms, 1000 rows, 16 + 8 heads of 128, f32: 47 ->
-// 7.5 us; 1000 rows, 4 + 1 heads of 256, f16: 43.8 -> 11.2 us (traced).
+// 12.5 us; 1000 rows, 4 + 1 heads of 256, f16: 43.8 -> 11.2 us (kernel trace).
 // (kMaxD: the largest head length, which sizes the LDS.)
 template <typename KV, uint32_t kMaxD>
 __global__ __launch_bounds__(256) void append_tile_kernel(const AppendArgs a) {
