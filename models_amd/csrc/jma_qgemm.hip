@@ -121,9 +121,12 @@ __device__ __forceinline__ void store_tile(const float16_t& acc, uint32_t b, uin
     if (ok(e)) out[at(e)] = mode != 0 ? acc[e] + add[e] : acc[e];
 }
 
-// Barrier once at most N of this wave's loads are in flight and its LDS writes are done.
+// Barrier once at most N of this wave's loads are in flight and its LDS writes are done. N is counted
+// from the source, so it holds only while the compiler emits at least that many loads a step:
+// tests/test_product_waits_cpu.py plays the emitted loads and waits of every instance.
 template <int N>
 __device__ __forceinline__ void wait_barrier() {
+  static_assert(N >= 0 && N < 64, "the load counter has six bits");
   __builtin_amdgcn_s_waitcnt((N & 15) | (7 << 4) | (15 << 8) | ((N >> 4) << 14));
   asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
 }
