@@ -132,7 +132,11 @@ JMODELS_ATTN_API jmodels_attn_context* jmodels_attn_context_create(int32_t devic
 /* RS:521-537 analogue; NULL_POINTER for NULL. Destroys nothing else: KV caches and RoPE tables
  * must be destroyed first. */
 JMODELS_ATTN_API int32_t jmodels_attn_context_destroy(jmodels_attn_context* ctx);
-/* Waits for the context stream and reports errors recorded by kernels since the last call. */
+/* Waits for the context stream and for the device's null stream, and reports errors recorded by
+ * kernels since the last call. The context stream is a non-blocking one: no other call of this
+ * library orders it with the null stream, so a fill or copy made there (hipMemset may return before
+ * the device has written) is waited for, here or by the caller, before a call that reads or
+ * overwrites its memory. */
 JMODELS_ATTN_API int32_t jmodels_attn_context_synchronize(jmodels_attn_context* ctx);
 /* The context's hipStream_t, for callers that order their own work (events, copies) with it. */
 JMODELS_ATTN_API int32_t jmodels_attn_context_stream(jmodels_attn_context* ctx, void** stream_out);

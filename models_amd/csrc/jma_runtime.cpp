@@ -1060,7 +1060,11 @@ int32_t jmodels_attn_context_synchronize(jmodels_attn_context* ctx) {
   return guard([&] {
     check_ctx(ctx);
     set_device(ctx);
-    collect_errors(ctx);
+    hip_check(hipStreamSynchronize(ctx->stream), "hipStreamSynchronize");
+    // The context's stream does not wait for the null stream: a caller's fills and copies there, which
+    // may return early, are over with this call too.
+    hip_check(hipStreamSynchronize(nullptr), "hipStreamSynchronize");
+    raise_errors(ctx);
   });
 }
 

@@ -98,6 +98,19 @@ void run_op(const Op& op) {
   }
 }
 
+// Fills on the null stream run when something waits for that stream (the device may not have written
+// when hipMemset returns, and the library's stream, a non-blocking one, does not wait for it).
+std::vector<Op> g_null;
+
+void drain_null() {
+  std::vector<Op> ops;
+  {
+    std::lock_guard<std::mutex> l(g_mu);
+    ops.swap(g_null);
+  }
+  for (const Op& op : ops) run_op(op);
+}
+
 // At exit: a summary line, and exit status 86 when any check failed.
 struct Summary {
   Summary() {
@@ -137,6 +150,7 @@ hipError_t hipMalloc(void** ptr, size_t size) {
 
 hipError_t hipFree(void* ptr) {
   if (!ptr) return hipSuccess;
+  drain_null();
   {
     std::lock_guard<std::mutex> l(g_mu);
     auto it = g_live.find((uintptr_t)ptr);
@@ -151,6 +165,7 @@ hipError_t hipFree(void* ptr) {
 }
 
 hipError_t hipMemcpy(void* dst, const void* src, size_t bytes, hipMemcpyKind kind) {
+  drain_null();
   run_copy(dst, src, bytes, kind);
   return hipSuccess;
 }
@@ -165,6 +180,7 @@ hipError_t hipMemcpyAsync(void* dst, const void* src, size_t bytes, hipMemcpyKin
     s->ops.push_back(op);
     return hipSuccess;
   }
+  if (!s) drain_null();
   run_copy(dst, src, bytes, kind);
   return hipSuccess;
 }
@@ -179,7 +195,8 @@ hipError_t hipMemset(void* dst, int value, size_t bytes) {
   op.dst = dst;
   op.value = value;
   op.bytes = bytes;
-  run_op(op);
+  std::lock_guard<std::mutex> l(g_mu);
+  g_null.push_back(op);
   return hipSuccess;
 }
 
@@ -189,7 +206,13 @@ hipError_t hipMemsetAsync(void* dst, int value, size_t bytes, hipStream_t s) {
     error("hipMemsetAsync %s recorded into a graph%s", "", "");
     return hipErrorStreamCaptureUnsupported;
   }
-  return hipMemset(dst, value, bytes);
+  if (!s) return hipMemset(dst, value, bytes);
+  Op op{Op::kSet};
+  op.dst = dst;
+  op.value = value;
+  op.bytes = bytes;
+  run_op(op);
+  return hipSuccess;
 }
 
 hipError_t hipSetDevice(int device) { return device == 0 ? hipSuccess : hipErrorInvalidDevice; }
@@ -221,8 +244,14 @@ hipError_t hipStreamDestroy(hipStream_t stream) {
   return hipSuccess;
 }
 
-hipError_t hipStreamSynchronize(hipStream_t) { return hipSuccess; }
-hipError_t hipDeviceSynchronize(void) { return hipSuccess; }
+hipError_t hipStreamSynchronize(hipStream_t s) {
+  if (!s) drain_null();
+  return hipSuccess;
+}
+hipError_t hipDeviceSynchronize(void) {
+  drain_null();
+  return hipSuccess;
+}
 
 hipError_t hipStreamIsCapturing(hipStream_t s, hipStreamCaptureStatus* status) {
   *status = s && s->capturing ? hipStreamCaptureStatusActive : hipStreamCaptureStatusNone;

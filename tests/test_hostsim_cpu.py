@@ -82,3 +82,27 @@ def test_default_bench_line(sim):
     other prefills and decode layers, C4, C5 and the projections, ending in the JSON line."""
     out = _bench(sim, "--steps", "2", "--warmup", "1", "--no-cpu", timeout=1500)
     assert '"metric"' in out and '"roofline"' in out
+
+
+def _python(env, code):
+    run = subprocess.run([sys.executable, "-c", code], cwd=ROOT, env=env, capture_output=True, text=True,
+                         timeout=300)
+    out = run.stdout + run.stderr
+    assert run.returncode == 0 and " 0 errors" in out, out[-4000:]
+    assert "AddressSanitizer" not in out and "runtime error" not in out, out[-4000:]
+    return run.stdout
+
+
+def test_synchronize_waits_for_null_stream_fills(sim):
+    """A caller's hipMemset on the null stream is over once jmodels_attn_context_synchronize returns:
+    the context's non-blocking stream alone would not wait for it."""
+    _python(sim, """
+import ctypes
+from models_amd import attention as A, hip_runtime as rt
+with A.HipAttentionLibrary(0) as hip:
+    d = rt.DeviceArray(64)
+    rt.check(rt.hip().hipMemset(d.ptr, 0, d.nbytes), "hipMemset")
+    assert any(ctypes.string_at(d.ptr, d.nbytes)), "the fill has not run yet"
+    hip.synchronize()
+    assert not any(ctypes.string_at(d.ptr, d.nbytes)), "the fill was not waited for"
+""")
