@@ -370,15 +370,23 @@ JMA_HD void qgemm_tile(uint32_t id, uint32_t tiles_w, uint32_t recip, uint32_t t
   }
 }
 
-// The workgroup tile (index of kQGemmShape) of a product launch: the largest once its tiles cover
-// half the compute units (1000 rows: 3072 outputs of 3072 inputs, 192 tiles, 68 us against 73 with
-// 64 x 64 tiles; 512 rows, 96 tiles, 46 against 39), else the small ones, 32 rows wide for batches
-// that fit.
+// The workgroup tile (index of kQGemmShape) of a product launch, of 4096 inputs in these times:
+// 32-row tiles for batches that fit them, however many outputs (32 rows: 2048 outputs, Q5_0, 55 us,
+// as 64 x 64 tiles; 16384 outputs 59 against 94 with 128 x 128 tiles; 128256 outputs 231 against 273,
+// Q4_K 112 against 203, Q5_K 139 against 310); else 64 x 64 tiles while they fit the compute units once
+// (64 rows, 16384 outputs, 256 tiles: Q5_0 57 us against 95, Q4_K 42 against 62); else the largest
+// once they cover half the units. (Twice as many 64 x 64 tiles as units are level with the large ones
+// or better in Q4_0 and Q4_K, 72 against 86 us and 57 against 63 at 128 x 16384, but slower in Q8_0
+// and Q5_K by up to 14%; 1024 of them are slower in each, 1.26 to 1.82 times.) Q6_K has one tile.
 inline uint32_t plan_qgemm(const uint32_t* rows, uint32_t count, uint32_t batch, uint32_t cus) {
-  uint64_t tiles = 0;
-  for (uint32_t i = 0; i < count; ++i) tiles += (rows[i] + 127u) / 128u;
-  if (tiles * ((batch + 127u) / 128u) * 2 >= cus) return 0;
-  return batch <= 32 ? 2 : 1;
+  if (batch <= 32) return 2;
+  uint64_t small = 0, large = 0;
+  for (uint32_t i = 0; i < count; ++i) {
+    small += (rows[i] + 63u) / 64u;
+    large += (rows[i] + 127u) / 128u;
+  }
+  if (small * ((batch + 63u) / 64u) <= cus) return 1;
+  return large * ((batch + 127u) / 128u) * 2 >= cus ? 0 : 1;
 }
 
 struct QMatPlan {

@@ -1,4 +1,5 @@
-// CPU bounds check of the quantized-projection launches (models_amd/csrc/jma_quant.hip), built
+// CPU bounds check of the quantized-projection launches (models_amd/csrc/jma_quant.hip and
+// models_amd/csrc/jma_qgemm.hip), built
 // with g++ and AddressSanitizer / UndefinedBehaviorSanitizer by tests/test_plan_cpu.py.
 //
 // For each call below it routes every weight format the way quantized_matmul_impl does and plans
@@ -407,9 +408,27 @@ void walk(const Call& c) {
   delete[] B.x;
 }
 
+// The product's tile: no batch of at most 32 rows pads its activation rows past 32, none of at most 64
+// past 64 while that many 64 x 64 tiles fit the compute units; large launches keep the large tile.
+void check_tiles() {
+  auto rows_b = [](uint32_t batch, uint32_t rows) {
+    return jma::qgemm_rows_b(jma::kQGemmShape[jma::plan_qgemm(&rows, 1, batch, 256)]);
+  };
+  for (uint32_t rows : {1u, 64u, 2048u, 16300u, 16384u, 20000u, 131072u})
+    for (uint32_t batch : {16u, 17u, 31u, 32u})
+      expect(rows_b(batch, rows) == 32, "32-row tiles: " + std::to_string(batch) + " x " + std::to_string(rows));
+  for (uint32_t rows : {1u, 64u, 2048u, 16300u, 16384u})
+    for (uint32_t batch : {33u, 48u, 64u})
+      expect(rows_b(batch, rows) == 64, "64-row tiles: " + std::to_string(batch) + " x " + std::to_string(rows));
+  expect(rows_b(64, 32768) == 128 && rows_b(65, 16384) == 128 && rows_b(1000, 3072) == 128 &&
+             rows_b(512, 3072) == 64 && rows_b(77, 2048) == 64,
+         "tiles of larger launches");
+}
+
 }  // namespace
 
 int main() {
+  check_tiles();
   const std::vector<Call> calls = {
       // decode shapes: Llama-3.2-1B Q/K/V and wo, Qwen2 with biases
       {"llama1b qkv decode", {1, 0, 0}, {2048, 512, 512}, 1, 2048, 0},
