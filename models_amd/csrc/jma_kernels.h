@@ -316,9 +316,9 @@ hipError_t launch_q8_0_quant(const float* x, uint32_t batch, uint32_t cols, void
 hipError_t launch_qgemm(const QMatArgs& a, uint32_t fmt, uint32_t shape, uint32_t tiles_w,
                         const void* act, const void* act_scale, hipStream_t stream);
 // The same for Q4_K (fmt 2), Q6_K (fmt 3) and Q5_K (fmt 4) on Q8_K activations, with the block's
-// 16-element sums (halves, qact_sum_index) and f32 scales; classes: the values in Q6_K's order
-// (qact_class_index), null when no weight of the call is Q6_K. A product reads act (Q6_K: the
-// values in its order), sums (not Q6_K) and scales.
+// 16-element sums (halves, qact_sum_index) and f32 scales; act null (the sums are not written either):
+// every weight of the call is Q6_K; classes: the values in Q6_K's order (qact_class_index), null: none
+// is. A product reads act (Q6_K: the values in its order), sums (not Q6_K) and scales.
 hipError_t launch_q8_k_quant(const float* x, uint32_t batch, uint32_t cols, void* act, void* classes,
                              void* sums, void* scales, hipStream_t stream);
 hipError_t launch_qkgemm(const QMatArgs& a, uint32_t fmt, uint32_t shape, uint32_t tiles_w,

@@ -305,28 +305,38 @@ JMA_HD uint64_t qact_sum_index(uint32_t b, uint32_t blk, uint32_t i, uint32_t KB
   return ((uint64_t)(b / 32u) * KB + blk) * 512u + (i / 8u) * 256u + (b % 32u) * 8u + i % 8u;
 }
 JMA_HD uint32_t qact_tiles(uint32_t batch) { return (batch + 31u) / 32u; }
-// Bytes of the activations of a batch (32-row tiles), rounded up to keep what follows aligned.
-JMA_HD uint64_t qact_bytes(uint32_t batch, uint32_t cols) {
-  return ((uint64_t)qact_tiles(batch) * 32u * cols * 2u + 255u) / 256u * 256u;
-}
-// Q8_K scratch: the activations in both orders, the sums, the scales, from its start.
-struct QactKOffsets {
-  uint64_t classes, sums, scales, total;
+// What a product call keeps of its activations in scratch, as offsets: the values (for any format but
+// Q6_K), the values in Q6_K's order, the 16-element sums (Q4_K, Q5_K) and the scales. 32-element
+// formats take 2 1/16 bytes per activation, Q4_K and Q5_K 2 9/64, Q6_K 2 1/64, a call of Q6_K and
+// others 4 9/64, with the batch rounded up to 32 rows.
+struct QactLayout {
+  uint64_t act, classes, sums, scales, total;
 };
-JMA_HD QactKOffsets qact_k_offsets(uint32_t batch, uint32_t cols) {
-  QactKOffsets o;
-  const uint64_t blocks = (uint64_t)qact_tiles(batch) * (cols / 256u);
-  o.classes = qact_bytes(batch, cols);
-  o.sums = 2u * o.classes;
-  o.scales = o.sums + blocks * 1024u;
-  o.total = o.scales + blocks * 32u * 4u;
+enum QactKind : uint32_t { kQactBlocks = 0, kQactK = 1, kQactQ6 = 2, kQactKAndQ6 = 3 };  // bits: Q4_K / Q5_K, Q6_K
+JMA_HD QactLayout qact_layout(uint64_t elements, uint32_t kind) {  // elements: 32-row tiles x cols
+  const auto up = [](uint64_t bytes) { return (bytes + 255u) / 256u * 256u; };
+  const uint64_t values = up(elements * 2u);
+  QactLayout o;
+  o.act = 0;
+  o.classes = kind == kQactQ6 ? 0 : values;
+  o.sums = o.classes + (kind & kQactQ6 ? values : 0);
+  o.scales = o.sums + (kind & kQactK ? up(elements / 8u) : 0);
+  o.total = o.scales + up(kind == kQactBlocks ? elements / 16u : elements / 64u);
   return o;
 }
-// Scratch to hold for calls of up to `elements` = batch x cols activations, whatever their format
-// and shape, so that a captured call no larger than an eager one before it never has to grow it:
-// rounding a batch of 16 or more up to 32 rows at most doubles it (two orders of 2-byte values:
-// 8 bytes per activation); sums and scales take at most 1/4 + 1/32 of a byte more.
-JMA_HD uint64_t qact_reserve_bytes(uint64_t elements) { return elements * 8u + elements / 2u + 4096u; }
+JMA_HD uint64_t qact_elements(uint32_t batch, uint32_t cols) { return (uint64_t)qact_tiles(batch) * 32u * cols; }
+// Scratch to hold after a call, so that a captured call of no more activations than an eager one before
+// it, of up to kQactMaxCols inputs, never has to grow it: rounding a batch up to 32 rows adds at most
+// 31 rows and, from 16 rows on, at most doubles it. Within kQactAnyKind bytes there is room for calls of any
+// kind; beyond, for those of this call's (and what a smaller kind leaves).
+constexpr uint64_t kQactMaxCols = 65536, kQactAnyKind = 64u << 20;
+JMA_HD uint64_t qact_reserve_bytes(uint32_t batch, uint32_t cols, uint32_t kind) {
+  const uint64_t n = (uint64_t)batch * cols, own = qact_elements(batch, cols);
+  const uint64_t others = n < 31u * kQactMaxCols ? 2u * n : n + 31u * kQactMaxCols;
+  const uint64_t elements = own > others ? own : others;
+  const uint64_t need = qact_layout(elements, kind).total, any = qact_layout(elements, kQactKAndQ6).total;
+  return any <= kQactAnyKind ? any : need > kQactAnyKind ? need : kQactAnyKind;
+}
 
 // Workgroup tiles of the product: 32 bt nb activation rows x 32 wt nw weight rows on nb x nw
 // waves of bt x wt 32 x 32 tiles each, half a weight block staged per thread and step.

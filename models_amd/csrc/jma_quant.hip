@@ -545,7 +545,7 @@ __global__ __launch_bounds__(kQThreads) void q8_0_quant_kernel(const float* x, u
 // Q8_K activations of the K-quants: a workgroup takes one 256-element block of 8 rows, 32 threads
 // a row with 8 elements each. Rows past the batch (up to a multiple of 32) get zeros. The block's
 // sixteen 16-element sums (below 2048 in magnitude, exact in f16) and its scale go beside them;
-// `classes` (null = not needed) gets the values in Q6_K's order too.
+// `classes` (null = not needed) gets the values in Q6_K's order too; act null: only that order.
 __global__ __launch_bounds__(kQThreads) void q8_k_quant_kernel(const float* x, uint32_t batch,
                                                                uint32_t cols, _Float16* act,
                                                                _Float16* classes, _Float16* sums,
@@ -561,8 +561,10 @@ __global__ __launch_bounds__(kQThreads) void q8_k_quant_kernel(const float* x, u
     s = 0;
     scale = 0.0f;
   }
-  *(half8_t*)(act + qact_index(b, blk * 256u + part * 8u, cols)) = act_run(packed);
-  if ((part & 1u) == 0) sums[qact_sum_index(b, blk, part / 2u, KB)] = (_Float16)(short)s;
+  if (act != nullptr) {
+    *(half8_t*)(act + qact_index(b, blk * 256u + part * 8u, cols)) = act_run(packed);
+    if ((part & 1u) == 0) sums[qact_sum_index(b, blk, part / 2u, KB)] = (_Float16)(short)s;
+  }
   if (part == 0) scales[qact_scale_index(b, blk, KB)] = scale;
   if (classes == nullptr) return;
   // The four lanes of a quad hold elements l, l + 8, l + 16, l + 24 of one 32-element run for every

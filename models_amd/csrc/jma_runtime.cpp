@@ -153,7 +153,7 @@ struct jmodels_attn_context {
   unsigned char* host = nullptr;
   int* err = nullptr;
   DeviceBuffer part_acc, part_ml, part_f, counters, pf_part, pf_tickets, qrot, stage_q, stage_k, stage_v, stage_out;
-  DeviceBuffer qact;                // Q8_0 activations of prefill-sized projections
+  DeviceBuffer qact;                // quantized activations of prefill-sized projections
   DeviceBuffer pp_part, pp_tickets; // split stripe pairs of the head-dim-512 f16 prefill
   int decode_target_blocks = 512;   // workgroups a decode launch aims for (two per CU)
   int tiles_per_wave = 1;           // minimum tiles each decode wave streams
@@ -898,17 +898,19 @@ void quantized_matmul_impl(jmodels_attn_context* ctx, const std::vector<QuantMat
   const bool gemm = batch >= jma::kQGemmMinBatch;
   char* act = nullptr;
   char* act_scale = nullptr;
-  const jma::QactKOffsets ko = jma::qact_k_offsets(batch, cols);
+  uint32_t kind = jma::kQactBlocks;
+  for (const QuantMatrix& m : mats)
+    if (kq) kind |= m.format == JMODELS_ATTN_WEIGHTS_Q6_K ? jma::kQactQ6 : jma::kQactK;
+  const jma::QactLayout ko = jma::qact_layout(jma::qact_elements(batch, cols), kind);
   set_device(ctx);
   if (gemm) {
-    ctx->qact.reserve(jma::qact_reserve_bytes((uint64_t)batch * cols), ctx->stream, "projection activations");
+    ctx->qact.reserve(jma::qact_reserve_bytes(batch, cols, kind), ctx->stream, "projection activations");
     act = (char*)ctx->qact.ptr;
-    act_scale = act + (kq ? ko.scales : jma::qact_bytes(batch, cols));
-    bool q6 = false;
-    for (const QuantMatrix& m : mats) q6 |= m.format == JMODELS_ATTN_WEIGHTS_Q6_K;
+    act_scale = act + ko.scales;
     if (kq)
-      hip_check(jma::launch_q8_k_quant(input, batch, cols, act, q6 ? act + ko.classes : nullptr,
-                                       act + ko.sums, act_scale, ctx->stream),
+      hip_check(jma::launch_q8_k_quant(input, batch, cols, kind & jma::kQactK ? act : nullptr,
+                                       kind & jma::kQactQ6 ? act + ko.classes : nullptr, act + ko.sums,
+                                       act_scale, ctx->stream),
                 "activation quantization launch");
     else
       hip_check(jma::launch_q8_0_quant(input, batch, cols, act, act_scale, ctx->stream),

@@ -358,6 +358,13 @@ long hipsim_errors(void) {
   return g_errors;
 }
 
+size_t hipsim_live_bytes(void) {
+  std::lock_guard<std::mutex> l(g_mu);
+  size_t n = 0;
+  for (const auto& it : g_live) n += it.second;
+  return n;
+}
+
 long hipsim_launches(void) {
   std::lock_guard<std::mutex> l(g_mu);
   return g_launches;

@@ -239,9 +239,10 @@ hipError_t launch_q8_k_quant(const float* x, uint32_t batch, uint32_t cols, void
   Launch* l = new Launch();
   const size_t rows = (size_t)qact_tiles(batch) * 32;
   add(l, x, (size_t)batch * cols * 4, "activations");
-  add(l, act, rows * cols * 2, "quantized activations");
+  if (!act && !classes) hipsim_fail("quantized activations in neither order");
+  if (act) add(l, act, rows * cols * 2, "quantized activations");
   if (classes) add(l, classes, rows * cols * 2, "quantized activations in class order");
-  add(l, sums, rows * (cols / 16) * 2, "activation sums");
+  if (act) add(l, sums, rows * (cols / 16) * 2, "activation sums");
   add(l, scales, rows * (cols / 256) * 4, "activation scales");
   return submit(stream, "q8_k_quant_kernel", l);
 }

@@ -159,8 +159,9 @@ void walk_quant(const Call& c, Buffers& B) {
     expect(B.act[i] == 1 && B.act[i + 3] == 1 && B.act[i + 7] == 1, c.name + ": every activation run once");
   for (uint64_t i = 0; i < (uint64_t)rows * K; ++i)
     expect(B.act_scale[i] == 1, c.name + ": every activation scale once");
-  const uint64_t used = jma::qact_bytes(c.batch, c.cols) + (uint64_t)rows * K * 2;
-  expect(used <= jma::qact_reserve_bytes((uint64_t)c.batch * c.cols), c.name + ": activation scratch");
+  const jma::QactLayout o = jma::qact_layout(jma::qact_elements(c.batch, c.cols), jma::kQactBlocks);
+  expect(o.act == 0 && o.scales >= (uint64_t)rows * c.cols * 2 && o.total - o.scales >= (uint64_t)rows * K * 2,
+         c.name + ": activation scratch regions");
 }
 
 // qkgemm_kernel (Q4_K, Q5_K) and q6gemm_kernel (Q6_K): as walk_qgemm, a step one 32-element group
@@ -261,11 +262,16 @@ void walk_quant_k(const Call& c, Buffers& B) {
   for (uint64_t i = 0; i < (uint64_t)rows * KB * 16u; ++i) once &= B.act_sum[i] == 1;
   for (uint64_t i = 0; i < (uint64_t)rows * KB; ++i) once &= B.act_scale_k[i] == 1.0f;
   expect(once, c.name + ": every quantized activation, sum and scale once");
-  const jma::QactKOffsets o = jma::qact_k_offsets(c.batch, c.cols);
-  expect(o.classes >= (uint64_t)rows * c.cols * 2 && o.sums - o.classes >= (uint64_t)rows * c.cols * 2 &&
-             o.scales - o.sums >= (uint64_t)rows * KB * 32 && o.total - o.scales >= (uint64_t)rows * KB * 4,
-         c.name + ": activation scratch regions");
-  expect(o.total <= jma::qact_reserve_bytes((uint64_t)c.batch * c.cols), c.name + ": activation scratch");
+  const uint64_t values = (uint64_t)rows * c.cols * 2;
+  for (uint32_t kind : {jma::kQactK, jma::kQactQ6, jma::kQactKAndQ6}) {
+    const jma::QactLayout o = jma::qact_layout(jma::qact_elements(c.batch, c.cols), kind);
+    const uint64_t after_act = kind & jma::kQactK ? values : 0, after_classes = kind & jma::kQactQ6 ? values : 0;
+    expect(o.act == 0 && o.classes >= after_act && o.sums - o.classes >= after_classes &&
+               o.scales - o.sums >= (kind & jma::kQactK ? (uint64_t)rows * KB * 32 : 0) &&
+               o.total - o.scales >= (uint64_t)rows * KB * 4 && o.classes % 16 == 0 && o.sums % 16 == 0 &&
+               o.scales % 16 == 0,
+           c.name + ": activation scratch regions");
+  }
 }
 
 // qmatvec_kernel / qkmatvec_kernel: the tile's weight units, the activation rows of each pass,
@@ -425,10 +431,30 @@ void check_tiles() {
          "tiles of larger launches");
 }
 
+// Scratch of a product call: enough for itself and for any of at most as many activations (up to 65536
+// inputs) of its kind; from 64 MiB on no more than its kind needs, with 31 rows of 65536 inputs to spare.
+void check_scratch() {
+  const uint32_t shapes[][2] = {{16, 256}, {17, 4096}, {31, 65536}, {77, 2048}, {1000, 3072}, {2048, 8192}, {4096, 8192}, {16384, 8192}};
+  for (uint32_t kind = 0; kind < 4; ++kind)
+    for (const auto& a : shapes) {
+      const std::string at = "scratch of " + std::to_string(a[0]) + " x " + std::to_string(a[1]) + ", kind " + std::to_string(kind);
+      const uint64_t held = jma::qact_reserve_bytes(a[0], a[1], kind), n = (uint64_t)a[0] * a[1];
+      for (uint32_t cols = 256; cols <= 65536; cols += 256) {
+        const uint64_t batch = n / cols;
+        if (batch < jma::kQGemmMinBatch) break;
+        const uint64_t need = jma::qact_layout(jma::qact_elements((uint32_t)batch, cols), kind).total;
+        expect(need <= held, at + ": room for " + std::to_string(batch) + " x " + std::to_string(cols));
+      }
+      const uint64_t per64 = kind == 0 ? 132 : kind == 1 ? 137 : kind == 2 ? 129 : 265;  // bytes per 64 activations
+      expect(held <= std::max<uint64_t>(64u << 20, (n + 31 * 65536) * per64 / 64 + 4096), at + ": no more than its kind needs");
+    }
+}
+
 }  // namespace
 
 int main() {
   check_tiles();
+  check_scratch();
   const std::vector<Call> calls = {
       // decode shapes: Llama-3.2-1B Q/K/V and wo, Qwen2 with biases
       {"llama1b qkv decode", {1, 0, 0}, {2048, 512, 512}, 1, 2048, 0},

@@ -106,3 +106,38 @@ with A.HipAttentionLibrary(0) as hip:
     hip.synchronize()
     assert not any(ctypes.string_at(d.ptr, d.nbytes)), "the fill was not waited for"
 """)
+
+
+def test_projection_scratch(sim):
+    """A prefill-sized projection holds scratch for what its formats keep of the activations (Q8_0 2 1/16
+    bytes each, Q6_K alone 2 1/64, with 31 rows of 65536 inputs to spare), and a captured call of no
+    more activations than the eager one before it does not have to grow it."""
+    _python(sim, """
+import ctypes
+import numpy as np
+from models_amd import attention as A, hip_runtime as rt
+live = rt.hip().hipsim_live_bytes
+live.restype = ctypes.c_size_t
+sizes = {A.WEIGHTS_Q8_0: (34, 32), A.WEIGHTS_Q4_K: (144, 256), A.WEIGHTS_Q6_K: (210, 256)}
+
+def call(hip, formats, batch, cols, x, out):
+    ws = [rt.DeviceArray(cols // sizes[f][1] * sizes[f][0], np.uint8) for f in formats]
+    hip.quantized_grouped_matmul_device(formats, [w.ptr for w in ws], [w.nbytes for w in ws], [1] * len(ws),
+                                        x.ptr, x.count, out.ptr, out.count, batch, cols)
+
+n, spare = 4096 * 8192, 31 * 65536
+x, out = rt.DeviceArray(n), rt.DeviceArray(4 * 4096)
+for fmt, per in ((A.WEIGHTS_Q8_0, 2 + 1 / 16), (A.WEIGHTS_Q4_K, 2 + 9 / 64), (A.WEIGHTS_Q6_K, 2 + 1 / 64)):
+    with A.HipAttentionLibrary(0) as hip:
+        before = live()
+        call(hip, [fmt], 4096, 8192, x, out)
+        held = live() - before
+        assert n * per <= held <= max((n + spare) * per + 4096, 64 << 20), (fmt, held / n)
+small = rt.DeviceArray(32 * 4096)
+with A.HipAttentionLibrary(0) as hip:
+    call(hip, [A.WEIGHTS_Q8_0], 32, 4096, small, out)
+    before = live()
+    call(hip, [A.WEIGHTS_Q4_K, A.WEIGHTS_Q6_K], 16, 8192, small, out)
+    call(hip, [A.WEIGHTS_Q6_K], 17, 7680, small, out)
+    assert live() == before, "a call of no more activations grew the scratch"
+""")
