@@ -399,6 +399,12 @@ inline uint32_t plan_qgemm(const uint32_t* rows, uint32_t count, uint32_t batch,
   return large * ((batch + 127u) / 128u) * 2 >= cus ? 0 : 1;
 }
 
+// Threads of a product launch over tiles_w weight tiles; one launch holds fewer than 2^32.
+inline uint64_t qgemm_launch_threads(uint32_t fmt, uint32_t shape, uint64_t tiles_w, uint32_t batch) {
+  const QGemmShape s = qgemm_shape(fmt, shape);
+  return tiles_w * ((batch + (uint64_t)qgemm_rows_b(s) - 1) / qgemm_rows_b(s)) * qgemm_threads(s);
+}
+
 struct QMatPlan {
   uint32_t rows_per_tile = 0, chunk = 0;  // 0: cols too large for one workgroup's LDS
 };

@@ -845,8 +845,8 @@ struct QuantMatrix {
 };
 
 // Checks a quantized projection call the way backend-native checks its batched matmuls
-// (RS:1017-1060: null pointers, shape, buffer sizes), then launches it: activation rows in chunks
-// that fit one workgroup's LDS, one launch per chunk and weight format.
+// (RS:1017-1060: null pointers, shape, buffer sizes), then launches it: one launch per weight format,
+// before it one that quantizes the activations of a prefill-sized batch.
 void quantized_matmul_impl(jmodels_attn_context* ctx, const std::vector<QuantMatrix>& mats,
                            const float* input, uint64_t input_elements, float* output,
                            uint64_t output_elements, uint32_t batch, uint32_t cols,
@@ -902,6 +902,32 @@ void quantized_matmul_impl(jmodels_attn_context* ctx, const std::vector<QuantMat
   for (const QuantMatrix& m : mats)
     if (kq) kind |= m.format == JMODELS_ATTN_WEIGHTS_Q6_K ? jma::kQactQ6 : jma::kQactK;
   const jma::QactLayout ko = jma::qact_layout(jma::qact_elements(batch, cols), kind);
+  // Rows of one format's matrices, and the tile of its product.
+  struct FormatRows {
+    uint32_t rows[jma::kQMaxMatrices], count = 0;
+  };
+  auto rows_of = [&](uint32_t fmt) {
+    FormatRows r;
+    for (const QuantMatrix& m : mats)
+      if (m.format == fmt) r.rows[r.count++] = m.rows;
+    return r;
+  };
+  if (gemm) {
+    // Refused before anything is enqueued: batches past 4194240 rows (the calls' limit since they ran
+    // as rows of 65535 64-row tiles) and grids past one launch.
+    bool fits = (batch + 63u) / 64u <= 65535u;
+    for (uint32_t fmt = 0; fmt <= JMODELS_ATTN_WEIGHTS_Q5_0; ++fmt) {
+      const FormatRows r = rows_of(fmt);
+      if (r.count == 0) continue;
+      const uint32_t shape = jma::plan_qgemm(r.rows, r.count, batch, ctx->cus);
+      const uint32_t R = jma::qgemm_rows_w(jma::qgemm_shape(fmt, shape));
+      uint64_t tiles = 0;
+      for (uint32_t i = 0; i < r.count; ++i) tiles += ((uint64_t)r.rows[i] + R - 1) / R;
+      fits = fits && jma::qgemm_launch_threads(fmt, shape, tiles, batch) <= 0xFFFFFFFFu;
+    }
+    require(fits, JMODELS_ATTN_INVALID_SHAPE,
+            "batch_size or rows too large for one projection launch: " + std::to_string(batch));
+  }
   set_device(ctx);
   if (gemm) {
     ctx->qact.reserve(jma::qact_reserve_bytes(batch, cols, kind), ctx->stream, "projection activations");
@@ -925,11 +951,9 @@ void quantized_matmul_impl(jmodels_attn_context* ctx, const std::vector<QuantMat
             "cols too large for the device projection: " + std::to_string(cols));
   }
   for (uint32_t fmt = 0; fmt <= JMODELS_ATTN_WEIGHTS_Q5_0; ++fmt) {
-    uint32_t fmt_rows[jma::kQMaxMatrices], count = 0;
-    for (const QuantMatrix& m : mats)
-      if (m.format == fmt) fmt_rows[count++] = m.rows;
-    if (count == 0) continue;
-    const uint32_t shape = gemm ? jma::plan_qgemm(fmt_rows, count, batch, ctx->cus) : 0u;
+    const FormatRows r = rows_of(fmt);
+    if (r.count == 0) continue;
+    const uint32_t shape = gemm ? jma::plan_qgemm(r.rows, r.count, batch, ctx->cus) : 0u;
     const uint32_t R = gemm ? jma::qgemm_rows_w(jma::qgemm_shape(fmt, shape)) : qp.rows_per_tile;
     jma::QMatArgs a{};
     a.x = input;
@@ -954,8 +978,6 @@ void quantized_matmul_impl(jmodels_attn_context* ctx, const std::vector<QuantMat
       out_off += (uint64_t)batch * m.rows;
     }
     if (gemm) {
-      require((batch + 63u) / 64u <= 65535u, JMODELS_ATTN_INVALID_SHAPE,
-              "batch_size too large for one projection launch: " + std::to_string(batch));
       if (kq)
         hip_check(jma::launch_qkgemm(a, fmt, shape, tiles, fmt == JMODELS_ATTN_WEIGHTS_Q6_K ? act + ko.classes : act,
                                      act + ko.sums, act_scale, ctx->stream),

@@ -141,3 +141,26 @@ with A.HipAttentionLibrary(0) as hip:
     call(hip, [A.WEIGHTS_Q6_K], 17, 7680, small, out)
     assert live() == before, "a call of no more activations grew the scratch"
 """)
+
+
+def test_projection_past_one_launch_is_refused_first(sim):
+    """A product whose grid would pass 2^32 threads, or whose batch the calls' limit, is refused as an
+    invalid shape before its activations are quantized. (The buffers' claimed sizes pass the size checks;
+    nothing is ever read from them.)"""
+    _python(sim, """
+import ctypes
+from models_amd import attention as A, hip_runtime as rt
+launches = rt.hip().hipsim_launches
+launches.restype = ctypes.c_long
+x = rt.DeviceArray(64 * 32)
+with A.HipAttentionLibrary(0) as hip:
+    for batch, rows in ((16, 0xFFFFFF00), (64, 0xFFFFFF00), (65535 * 64 + 1, 32)):
+        try:
+            hip.quantized_matmul_device(A.WEIGHTS_Q4_0, x.ptr, rows * 18, x.ptr, batch * 32, x.ptr, batch * rows,
+                                        batch, rows, 32)
+        except A.AttentionStatusError as e:
+            assert "INVALID_SHAPE" in str(e), e
+        else:
+            raise AssertionError("not refused")
+        assert launches() == 0
+""")
