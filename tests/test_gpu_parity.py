@@ -1003,6 +1003,9 @@ PREFILL_TILE_CASES = {
     "rotated-in-kernel": (True, 12, 4, 128, 128, True, False, 0, 1001),
     "rotated-in-kernel-interleaved-chunk": (True, 12, 4, 64, 64, False, False, 45, 701),
     "rotated-in-kernel-partial": (True, 16, 2, 256, 128, False, False, 31, 513),
+    "rotated-in-kernel-d256": (True, 16, 2, 256, 256, True, False, 7, 513),
+    "rotated-in-kernel-d32": (True, 32, 8, 32, 32, True, False, 3, 300),
+    "rotated-in-kernel-d32-interleaved": (True, 32, 8, 32, 32, False, False, 0, 257),
     "at-the-rule": (True, 32, 8, 64, 64, True, False, 0, 256),
     "below-the-rule": (True, 32, 8, 64, 64, True, False, 0, 255),
     "neox-partial": (True, 32, 8, 128, 64, True, False, 1, 600),
@@ -1052,6 +1055,51 @@ def test_prefill_by_cache_tiles_equals_rows(hip, case):
         rope.close()
         if norm is not None:
             norm.close()
+
+
+ROTATED_PREFILL_CASES = [
+    # (heads, KV heads, d, NeoX pairs, window, ring slots or 0, JMA_PREFILL_SPLIT_TILES, first position, rows)
+    (12, 4, 128, True, 200, 0, "2", 90, 701),
+    (12, 4, 128, True, 200, 960, "2", 1500, 701),
+    (32, 8, 64, False, 130, 448, "0", 1000, 300),
+    (32, 8, 64, True, 0, 0, "2", 0, 300),
+    (16, 2, 256, True, 512, 0, "2", 100, 513),
+    (16, 2, 256, False, 96, 640, "2", 700, 515),
+]
+
+
+@pytest.mark.parametrize("case", ROTATED_PREFILL_CASES, ids=lambda c: "-".join(map(str, c)))
+def test_rotated_prefill_windows_rings_and_splits(monkeypatch, case):
+    """f16 prefills that rotate their queries in the kernel, with windows, on rings that wrap and with
+    their blocks split: the outputs of attend_causal on rotated queries, bit for bit, twice over the same
+    scratch (both run the same plan)."""
+    hq, hkv, d, neox, window, ring, split, start, n = case
+    assert n * hq >= 8192
+    total = start + n
+    q = normal(23, f"rp/{case}/q", (n, hq * d))
+    k = normal(23, f"rp/{case}/k", (total, hkv * d))
+    v = normal(23, f"rp/{case}/v", (total, hkv * d))
+    monkeypatch.setenv("JMA_PREFILL_SPLIT_TILES", split)
+    with A.HipAttentionLibrary(0) as lib:
+        rope = lib.rotary_table(d, 1e6, 1.0, max_positions=total)
+        a, b = (lib.layered_kv_cache([A.LayerSpec(hkv, d, d, ring)], total, half_precision=True) for _ in range(2))
+        try:
+            layer = A.AttentionLayer(0, hq, sliding_window=window, neox=neox, rope=rope)
+            store = A.AttentionLayer(0, hkv, sliding_window=window, neox=neox, rope=rope)
+            for kv in (a, b):
+                if start:
+                    kv.append(store, np.arange(start), k[:start], k[:start], v[:start])
+            q_rot = np.empty_like(q)
+            for part in (slice(0, n, 2), slice(1, n, 2)):  # lists of positions, never a run of them
+                at = np.arange(n)[part]
+                q_rot[part] = b.append(layer, start + at, q[part], k[start + at], v[start + at]).reshape(len(at), -1)
+            want = b.attend_causal(layer, start, q_rot)
+            for _ in range(2):
+                np.testing.assert_array_equal(a.prefill(layer, start, q, k[start:], v[start:]), want)
+        finally:
+            a.close()
+            b.close()
+            rope.close()
 
 
 @pytest.mark.parametrize("sessions", [1, 21, 22])

@@ -278,11 +278,12 @@ def test_prefill_sized_grouped_projection_with_addends(hip, mode):
 
 
 MATRIX_PRODUCT_EDGES = [
-    # (activation rows, weight rows, 256-element blocks of inputs): each workgroup tile of the
-    # product one short of, at and past its edges, and the fewest inputs it takes.
+    # (activation rows, weight rows, 256-element blocks of inputs, 96 inputs less for the 32-element
+    # formats): each workgroup tile of the product one short of, at and past its edges.
     (16, 1, 1), (31, 127, 2), (32, 128, 1), (33, 129, 1),      # 32 x 128 tiles, then 64 x 64
     (63, 63, 3), (65, 65, 2),
     (1281, 1537, 1), (1279, 1535, 2),                          # 128 x 128 (Q5_K and Q6_K 128 x 64)
+    (32, 16385, 1), (64, 16384, 1), (64, 16385, 1),            # wide outputs: 32 x 128, 64 x 64, 128 x 128
 ]
 
 
@@ -311,6 +312,19 @@ def test_matrix_product_tile_edges_bit_exact(hip, fmt, batch, rows, blocks):
             d.free()
     want = (oracle.quantized_matmul(fmt, w, x, batch, rows, cols) + resid).astype(np.float32)
     _exact(got, want.reshape(batch, rows), f"fmt {fmt} {batch}x{rows}x{cols}")
+
+
+@pytest.mark.parametrize("fmt", [A.WEIGHTS_Q4_0, A.WEIGHTS_Q8_0, A.WEIGHTS_Q5_0])
+@pytest.mark.parametrize("batch", [16, 33, 129])
+@pytest.mark.parametrize("cols", [32, 64, 96, 128, 192])
+def test_matrix_product_few_blocks_bit_exact(hip, fmt, batch, cols):
+    """Products over one to six 32-element blocks: fewer than the three steps that the kernel loads ahead,
+    and every remainder of its four-step loop, whose last steps must add exactly 0."""
+    rows = 1537 if batch == 129 else 130
+    w = _weights(fmt, rows, cols, f"few/{fmt}/{cols}")
+    x = synth.normal(11, f"few/x/{batch}/{cols}", (batch, cols)) * 2.0
+    got = hip.quantized_matmul(fmt, w, x, batch, rows, cols)
+    _exact(got, oracle.quantized_matmul(fmt, w, x, batch, rows, cols), f"fmt {fmt} {batch}x{rows}x{cols}")
 
 
 @pytest.mark.parametrize("case", ["q5_0-q8_0-q4_0 bias x300", "q8_0 wo residual x64",
