@@ -350,7 +350,11 @@ hipError_t launch_append(const AppendArgs& a, bool f16, hipStream_t stream) {
   const auto aligned = [](const void* p) { return ((uintptr_t)p & 15u) == 0; };
   const uint32_t max_d = std::max(a.dk, a.dv), units = (a.q_out ? a.num_heads : 0u) + 2 * a.num_kv_heads;
   // Without a norm to form, short launches are as fast or faster with a thread per pair (77 rows of
-  // 32 + 8 heads of 64: 11.5 against 12.3 us a prefill; 300 rows of keys and values 15.2 against 14.7).
+  // 32 + 8 heads of 64: 11.5 against 12.3 us a prefill; 300 rows of keys and values 15.2 against 14.7;
+  // 32 rows of 64 + 8 heads of 128 15.9 against 17.2; with as many KV heads as heads the tiles win from
+  // 128 rows, 32 + 32 heads of 128 20.6 against 18.6). With a norm the tiles win at any length (8 rows: 16 + 8
+  // heads of 128 16.0 against 10.9 us a prefill, 8 + 1 of 512 46.0 against 21.3; 2 rows 15.9 against 10.6):
+  // the line there lies higher than it need.
   const bool norms = a.q_norm_w || a.k_norm_w || a.v_norm;
   const uint32_t min_rows = norms ? 8u : a.q_out ? 512u : 256u;
   if (a.rows.contiguous && a.rows.count >= min_rows && a.pairs % 4 == 0 && a.dk % 16 == 0 && a.dv % 16 == 0 &&

@@ -275,7 +275,10 @@ constexpr uint32_t kQMatMaxChunk = 8;        // activation rows per pass
 constexpr uint32_t kQMatTargetBlocks = 1024;  // workgroups a projection launch aims for
 
 // Batches of at least kQGemmMinBatch activation rows run as a matrix product on the matrix cores
-// (jma_qgemm.hip) over activations quantized once into scratch.
+// (jma_qgemm.hip) over activations quantized once into scratch. The line is right for the square
+// projections of small models (2048 x 2048, 15 rows: Q4_0 15 us in the matrix-vector kernel against 27, Q4_K
+// 19 against 23); matrices of 4096 x 4096 cross between 8 and 15 rows (Q4_K 48 against 39 us at 8, Q4_0
+// 64 against 48 at 15), and wide outputs gain from 2 rows on (28672 x 4096, 15 rows: Q4_0 409 against 51).
 constexpr uint32_t kQGemmMinBatch = 16;
 
 // Quantized activations of a product, as halves (the int8 values exactly) in the order the matrix

@@ -151,9 +151,10 @@ __device__ __forceinline__ void static_for(F&& f) {
 //
 // What bounds it: per 32 x 32 tile and step 96 cycles of matrix ops (two for the dot, one for the
 // scale products, which on the vector unit would take 64 cycles more) and 64 of fma, plus the
-// unpacking, on one SIMD; the two overlap only partly (matrix unit busy 30% of the time, vector
-// issue about 40%). 3072 + 1024 + 1024 rows of 3072 inputs, 2048 activation rows, Q4_0: 519 us
-// with integer dots on the vector unit, 140 us with this kernel (459 TOPS).
+// unpacking, on one SIMD; the two overlap only partly (counters: matrix unit busy 38% of the compute
+// units' busy time, vector issue 50%, LDS 28%; waves wait for loads or barriers a quarter of their
+// time). 5120 weight rows of 3072 inputs, 2048 activation rows, kernel trace: Q4_0 552 us with integer
+// dots on the vector unit, 150 us with this kernel (429 TOPS); Q8_0 554 -> 157; Q5_0 171.
 template <int FMT, int BT, int WT, int NB, int NW>
 __global__ __launch_bounds__(64 * NB * NW, 2) void qgemm_kernel(const QMatArgs a, const _Float16* act,
                                                                  const uint16_t* act_scale,
@@ -326,9 +327,12 @@ __device__ __forceinline__ void dma4(const void* base, void* lds, uint32_t voff,
 // op each (16 inputs: the block's sums). qsum = fma(C, ssum, .) then rounds once, as the integer's
 // conversion does; Q5_K adds its two parts as integers.
 //
-// Measured (3072 + 1024 + 1024 rows of 3072 inputs, 2048 activation rows, Q4_K): 477 us with integer
-// dots on the vector unit, 117 us (550 TOPS) here; bound by operand reads from LDS (256 cycles a
-// step of a 128 x 128 tile) beside the matrix ops (256 a step on each SIMD).
+// Measured (5120 weight rows of 3072 inputs, 2048 activation rows, kernel trace): Q4_K 508 us with
+// integer dots on the vector unit, 118 us (547 TOPS) here; Q5_K 166 us. Per step of a 128 x 128 tile 256
+// cycles of matrix ops on each SIMD beside 256 of operand reads from LDS; by counters neither fills the
+// time (Q4_K: matrix unit busy 36% of the compute units' busy time, vector issue 48%, LDS 38%, a
+// quarter of that bank conflicts; Q5_K, with 1.6 times the LDS accesses and 2.3 times the vector work per
+// matrix op in its smaller tile: 21, 63 and 38%).
 //
 // Steps, buffers and loads as qgemm_kernel's, a step one 32-element group; the 4-bit quants of a
 // pair of groups are loaded once, the block's header one block ahead.
@@ -581,8 +585,9 @@ __global__ __launch_bounds__(64 * NB * NW, 2) void qkgemm_kernel(
 // integer of at most 32 * 4096 * 127 < 2^24. A step is one class of a block (32 elements of every
 // row); the activations come in class order (qact_class_index). Eight waves of one 32 x 32 tile,
 // each output with its eight chains; otherwise the steps, buffers and loads of qgemm_kernel. The
-// call of qkgemm_kernel's note with Q6_K weights: 907 us on the vector unit, 226 us here, bound by
-// the vector work (splitting the weights, 16 fma per tile and class) beside 4 matrix ops a class.
+// call of qkgemm_kernel's note with Q6_K weights: 917 us on the vector unit, 234 us here: splitting the
+// weights and 16 fma per tile and class beside 4 matrix ops a class, with waits between (counters:
+// matrix unit 25% of the busy time, vector issue 38%, LDS 45%, two fifths of that bank conflicts).
 __global__ __launch_bounds__(64 * kQ6KShape.nb * kQ6KShape.nw, 2) void q6gemm_kernel(
     const QMatArgs a, const _Float16* act, const float* scales, uint32_t tiles_w, uint32_t tiles_w_recip,
     uint32_t total) {

@@ -800,8 +800,11 @@ T* stage(DeviceBuffer& buf, const T* host, uint64_t elems, hipStream_t stream) {
 
 // A small host-buffer call's inputs and output in the context's host memory: the kernel reads and
 // writes them over the bus, which takes less than a copy each way (one layer-step of 16 + 8 heads of
-// 128 at 512 positions: 63 us with three copies in, one out and one of the error word; see the
-// sizes below for where the copies are better again).
+// 128 at 512 positions: 57.5 -> 26.5 us; what fell away: three copies in, one out and one of the error
+// word). Every split's workgroup reads its queries over the bus, twice with a norm: 32 + 8 heads of 128
+// with one at 65 000 positions still take 62 us against 96 with copies, 4 rows of 32 + 8 heads of 64
+// (48 KB in, 32 out) 25 against 60, the two-launch decode with a norm 34 against 67. No call of these sizes was
+// slower than with copies; larger blocks were not tried.
 constexpr size_t kHostErr = 256, kHostIn = 64 << 10, kHostOut = 64 << 10;
 constexpr size_t kHostBytes = kHostErr + kHostIn + kHostOut;
 
