@@ -361,10 +361,10 @@ JMODELS_ATTN_API int32_t jmodels_attn_prefill_device(jmodels_attn_context* ctx, 
  * Batches of 16 activation rows and more run as a matrix-core product on activations
  * quantized once into the context's scratch (the same bits as the matrix-vector path); such a
  * call made while the stream is captured returns NOT_CAPTURABLE when that scratch must grow first
- * (make the call once outside the capture). The scratch takes up to 2.2 bytes per activation (4.2 where a
- * call mixes Q6_K with Q4_K or Q5_K), with up to 31 rows of 65536 inputs to spare, and at least what
- * any call of as many activations needs up to 64 MiB; the context keeps it. Smaller batches use no
- * scratch memory.
+ * (make the call once outside the capture). The context keeps 2.1 bytes per activation of the largest
+ * call, 4.2 of a call of K-quants, with up to 31 rows of 65536 inputs to spare, so that calls of the same
+ * block size with no more activations need not grow it; where that cannot be allocated, what the call itself needs (at most
+ * 2.2, or 4.2 where it mixes Q6_K with Q4_K or Q5_K). Smaller batches use no scratch memory.
  *
  * Device pointers, asynchronous on the context stream. weights:
  * [rows][cols / 32 or cols / 256] blocks, 2-byte aligned; input [batch][cols] f32, 16-byte

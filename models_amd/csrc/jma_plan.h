@@ -328,17 +328,17 @@ JMA_HD QactLayout qact_layout(uint64_t elements, uint32_t kind) {  // elements: 
   return o;
 }
 JMA_HD uint64_t qact_elements(uint32_t batch, uint32_t cols) { return (uint64_t)qact_tiles(batch) * 32u * cols; }
-// Scratch to hold after a call, so that a captured call of no more activations than an eager one before
-// it, of up to kQactMaxCols inputs, never has to grow it: rounding a batch up to 32 rows adds at most
-// 31 rows and, from 16 rows on, at most doubles it. Within kQactAnyKind bytes there is room for calls of any
-// kind; beyond, for those of this call's (and what a smaller kind leaves).
+// Scratch to hold after a call where it can be had, so that a captured call of no more activations than
+// an eager one before it, of up to kQactMaxCols inputs, never has to grow it: rounding a batch up to 32
+// rows adds at most 31 rows and, from 16 rows on, at most doubles it. K-quant calls hold room for any
+// mix of them, 32-element calls for these, within kQactAnyKind bytes for K-quants too.
 constexpr uint64_t kQactMaxCols = 65536, kQactAnyKind = 64u << 20;
-JMA_HD uint64_t qact_reserve_bytes(uint32_t batch, uint32_t cols, uint32_t kind) {
+JMA_HD uint64_t qact_reserve_bytes(uint32_t batch, uint32_t cols, bool kq) {
   const uint64_t n = (uint64_t)batch * cols, own = qact_elements(batch, cols);
   const uint64_t others = n < 31u * kQactMaxCols ? 2u * n : n + 31u * kQactMaxCols;
   const uint64_t elements = own > others ? own : others;
-  const uint64_t need = qact_layout(elements, kind).total, any = qact_layout(elements, kQactKAndQ6).total;
-  return any <= kQactAnyKind ? any : need > kQactAnyKind ? need : kQactAnyKind;
+  const uint64_t blocks = qact_layout(elements, kQactBlocks).total, any = qact_layout(elements, kQactKAndQ6).total;
+  return kq || any <= kQactAnyKind ? any : blocks > kQactAnyKind ? blocks : kQactAnyKind;
 }
 
 // Workgroup tiles of the product: 32 bt nb activation rows x 32 wt nw weight rows on nb x nw

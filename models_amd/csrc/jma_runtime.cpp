@@ -62,12 +62,16 @@ int32_t guard(F&& body) {
 
 uint64_t round_up(uint64_t x, uint64_t m) { return (x + m - 1) / m * m; }
 
+bool capturing(hipStream_t stream) {
+  hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+  hip_check(hipStreamIsCapturing(stream, &status), "hipStreamIsCapturing");
+  return status != hipStreamCaptureStatusNone;
+}
+
 // Fails with NOT_CAPTURABLE when `stream` is being captured into a graph: a call that would
 // allocate, fill or wait there must first run once outside the capture.
 void require_not_capturing(hipStream_t stream, const char* what) {
-  hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
-  hip_check(hipStreamIsCapturing(stream, &status), "hipStreamIsCapturing");
-  if (status != hipStreamCaptureStatusNone)
+  if (capturing(stream))
     fail(JMODELS_ATTN_NOT_CAPTURABLE,
          std::string(what) + " needs more scratch memory than this context holds while its stream "
                              "is being captured; make the same call once outside the capture first");
@@ -80,16 +84,27 @@ void require_not_capturing(hipStream_t stream, const char* what) {
 struct DeviceBuffer {
   void* ptr = nullptr;
   size_t bytes = 0;
+  size_t not_had = SIZE_MAX;  // smallest preferred size that could not be allocated
   std::vector<void*> retired;
   // Growth is refused while `stream` is being captured; otherwise it waits for `stream` (its
-  // kernels may still use the old allocation, whose contents callers may copy).
-  void reserve(size_t need, hipStream_t stream, const char* what = "scratch") {
-    if (need <= bytes) return;
+  // kernels may still use the old allocation, whose contents callers may copy). `preferred`: what to
+  // hold where it can be had, so that later calls need not grow; only `need` is demanded.
+  void reserve(size_t need, hipStream_t stream, const char* what = "scratch", size_t preferred = 0) {
+    const size_t want = std::max(need, preferred);
+    if (want <= bytes) return;
+    if (need <= bytes && (want >= not_had || capturing(stream))) return;
     require_not_capturing(stream, what);
     hip_check(hipStreamSynchronize(stream), "hipStreamSynchronize");
-    const size_t grow = std::max({need, 2 * bytes, (size_t)1 << 16});
+    size_t grow = std::max({want, 2 * bytes, (size_t)1 << 16});
     void* fresh = nullptr;
-    hip_check(hipMalloc(&fresh, grow), "hipMalloc scratch");
+    hipError_t e = hipMalloc(&fresh, grow);
+    if (e == hipErrorOutOfMemory && grow > need) {
+      (void)hipGetLastError();
+      not_had = std::min(not_had, want);
+      if (need <= bytes) return;
+      e = hipMalloc(&fresh, grow = need);
+    }
+    hip_check(e, "hipMalloc scratch");
     if (ptr) retired.push_back(ptr);
     ptr = fresh;
     bytes = grow;
@@ -933,7 +948,7 @@ void quantized_matmul_impl(jmodels_attn_context* ctx, const std::vector<QuantMat
   }
   set_device(ctx);
   if (gemm) {
-    ctx->qact.reserve(jma::qact_reserve_bytes(batch, cols, kind), ctx->stream, "projection activations");
+    ctx->qact.reserve(ko.total, ctx->stream, "projection activations", jma::qact_reserve_bytes(batch, cols, kq));
     act = (char*)ctx->qact.ptr;
     act_scale = act + ko.scales;
     if (kq)

@@ -48,6 +48,7 @@ typedef struct hipDeviceProp_t {
 extern "C" {
 hipError_t hipMalloc(void** ptr, size_t size);
 hipError_t hipFree(void* ptr);
+hipError_t hipGetLastError(void);
 constexpr unsigned int hipHostMallocCoherent = 0x40000000u;
 hipError_t hipHostMalloc(void** ptr, size_t size, unsigned int flags);
 hipError_t hipHostFree(void* ptr);

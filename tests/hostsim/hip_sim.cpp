@@ -27,6 +27,7 @@ namespace {
 std::mutex g_mu;
 std::map<uintptr_t, size_t> g_live;  // base -> bytes
 long g_errors = 0, g_launches = 0;
+size_t g_largest = SIZE_MAX;  // larger allocations fail
 
 void error(const char* fmt, const char* a, const char* b = "") {
   ++g_errors;
@@ -139,6 +140,7 @@ extern "C" {
 
 hipError_t hipMalloc(void** ptr, size_t size) {
   if (!ptr) return hipErrorInvalidValue;
+  if (size > g_largest) return hipErrorOutOfMemory;
   void* p = nullptr;
   if (posix_memalign(&p, 256, size ? size : 1) != 0) return hipErrorOutOfMemory;
   memset(p, 0x5A, size);  // device memory starts undefined; never zero by accident
@@ -214,6 +216,8 @@ hipError_t hipMemsetAsync(void* dst, int value, size_t bytes, hipStream_t s) {
   run_op(op);
   return hipSuccess;
 }
+
+hipError_t hipGetLastError(void) { return hipSuccess; }
 
 hipError_t hipSetDevice(int device) { return device == 0 ? hipSuccess : hipErrorInvalidDevice; }
 
@@ -357,6 +361,8 @@ long hipsim_errors(void) {
   std::lock_guard<std::mutex> l(g_mu);
   return g_errors;
 }
+
+void hipsim_largest_allocation(size_t bytes) { g_largest = bytes; }
 
 size_t hipsim_live_bytes(void) {
   std::lock_guard<std::mutex> l(g_mu);

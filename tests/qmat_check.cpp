@@ -431,22 +431,25 @@ void check_tiles() {
          "tiles of larger launches");
 }
 
-// Scratch of a product call: enough for itself and for any of at most as many activations (up to 65536
-// inputs) of its kind; from 64 MiB on no more than its kind needs, with 31 rows of 65536 inputs to spare.
+// Scratch held after a product call: enough for itself and for any of at most as many activations (up to
+// 65536 inputs), of any kind of K-quants after one of them; from 64 MiB on no more than that, with 31 rows
+// of 65536 inputs to spare.
 void check_scratch() {
   const uint32_t shapes[][2] = {{16, 256}, {17, 4096}, {31, 65536}, {77, 2048}, {1000, 3072}, {2048, 8192}, {4096, 8192}, {16384, 8192}};
-  for (uint32_t kind = 0; kind < 4; ++kind)
+  for (bool kq : {false, true})
     for (const auto& a : shapes) {
-      const std::string at = "scratch of " + std::to_string(a[0]) + " x " + std::to_string(a[1]) + ", kind " + std::to_string(kind);
-      const uint64_t held = jma::qact_reserve_bytes(a[0], a[1], kind), n = (uint64_t)a[0] * a[1];
+      const std::string at = "scratch of " + std::to_string(a[0]) + " x " + std::to_string(a[1]) + (kq ? ", K" : "");
+      const uint64_t held = jma::qact_reserve_bytes(a[0], a[1], kq), n = (uint64_t)a[0] * a[1];
       for (uint32_t cols = 256; cols <= 65536; cols += 256) {
         const uint64_t batch = n / cols;
         if (batch < jma::kQGemmMinBatch) break;
-        const uint64_t need = jma::qact_layout(jma::qact_elements((uint32_t)batch, cols), kind).total;
-        expect(need <= held, at + ": room for " + std::to_string(batch) + " x " + std::to_string(cols));
+        for (uint32_t kind = 0; kind <= (kq ? 3u : 0u); ++kind) {
+          const uint64_t need = jma::qact_layout(jma::qact_elements((uint32_t)batch, cols), kind).total;
+          expect(need <= held, at + ": room for " + std::to_string(batch) + " x " + std::to_string(cols));
+        }
       }
-      const uint64_t per64 = kind == 0 ? 132 : kind == 1 ? 137 : kind == 2 ? 129 : 265;  // bytes per 64 activations
-      expect(held <= std::max<uint64_t>(64u << 20, (n + 31 * 65536) * per64 / 64 + 4096), at + ": no more than its kind needs");
+      const uint64_t per64 = kq ? 265 : 132;  // bytes per 64 activations
+      expect(held <= std::max<uint64_t>(64u << 20, (n + 31 * 65536) * per64 / 64 + 4096), at + ": no more than needed");
     }
 }
 

@@ -109,36 +109,63 @@ with A.HipAttentionLibrary(0) as hip:
 
 
 def test_projection_scratch(sim):
-    """A prefill-sized projection holds scratch for what its formats keep of the activations (Q8_0 2 1/16
-    bytes each, Q6_K alone 2 1/64, with 31 rows of 65536 inputs to spare), and a captured call of no
-    more activations than the eager one before it does not have to grow it."""
+    """A prefill-sized projection holds scratch for what its formats keep of the activations (32-element
+    formats 2 1/16 bytes each, K-quants up to 4 9/64, with 31 rows of 65536 inputs to spare), so that a
+    captured call of no more activations than the eager one before it does not have to grow it; where
+    so much cannot be allocated it takes what the call itself needs, and a captured call that fits runs."""
     _python(sim, """
 import ctypes
 import numpy as np
 from models_amd import attention as A, hip_runtime as rt
 live = rt.hip().hipsim_live_bytes
 live.restype = ctypes.c_size_t
-sizes = {A.WEIGHTS_Q8_0: (34, 32), A.WEIGHTS_Q4_K: (144, 256), A.WEIGHTS_Q6_K: (210, 256)}
+largest = lambda n: rt.hip().hipsim_largest_allocation(ctypes.c_size_t(n))
+Q8_0, Q4_K, Q6_K = A.WEIGHTS_Q8_0, A.WEIGHTS_Q4_K, A.WEIGHTS_Q6_K
+sizes = {Q8_0: (34, 32), Q4_K: (144, 256), Q6_K: (210, 256)}
 
-def call(hip, formats, batch, cols, x, out):
+def call(hip, formats, batch, cols):
     ws = [rt.DeviceArray(cols // sizes[f][1] * sizes[f][0], np.uint8) for f in formats]
     hip.quantized_grouped_matmul_device(formats, [w.ptr for w in ws], [w.nbytes for w in ws], [1] * len(ws),
                                         x.ptr, x.count, out.ptr, out.count, batch, cols)
 
+def captured(hip, *args):
+    g = rt.Graph(hip.stream(), lambda: call(hip, *args))
+    g.destroy()
+
 n, spare = 4096 * 8192, 31 * 65536
-x, out = rt.DeviceArray(n), rt.DeviceArray(4 * 4096)
-for fmt, per in ((A.WEIGHTS_Q8_0, 2 + 1 / 16), (A.WEIGHTS_Q4_K, 2 + 9 / 64), (A.WEIGHTS_Q6_K, 2 + 1 / 64)):
+x, out = rt.DeviceArray(n), rt.DeviceArray(4 * 8192)
+for fmt, per in ((Q8_0, 2 + 1 / 16), (Q4_K, 4 + 9 / 64), (Q6_K, 4 + 9 / 64)):
     with A.HipAttentionLibrary(0) as hip:
         before = live()
-        call(hip, [fmt], 4096, 8192, x, out)
+        call(hip, [fmt], 4096, 8192)
         held = live() - before
-        assert n * per <= held <= max((n + spare) * per + 4096, 64 << 20), (fmt, held / n)
-small = rt.DeviceArray(32 * 4096)
+        assert n * per <= held <= (n + spare) * per + 4096, (fmt, held / n)
+        if fmt != Q8_0:
+            call(hip, [Q4_K, Q6_K], 4096, 8192)
+            call(hip, [Q6_K, Q4_K], 4095, 8192)
+            call(hip, [Q4_K], 511, 65536)
+            assert live() - before == held, "a call of no more activations grew the scratch"
+for fmt, other, per in ((Q4_K, Q6_K, 2 + 9 / 64), (Q6_K, Q4_K, 2 + 1 / 64), (Q8_0, Q8_0, 2 + 1 / 16)):
+    with A.HipAttentionLibrary(0) as hip:
+        before = live()
+        largest(int(n * per) + 4096)  # not the whole preference
+        for _ in range(2):
+            call(hip, [fmt], 4096, 8192)
+            assert live() - before <= n * per + 4096, "more than the call itself needs"
+        captured(hip, [fmt], 4096, 8192)
+        if other != fmt:
+            try:
+                captured(hip, [fmt, other], 4096, 8192)
+                raise AssertionError("captured past its scratch")
+            except A.AttentionStatusError as e:
+                assert "NOT_CAPTURABLE" in str(e), e
+        largest(2 ** 62)
+x = rt.DeviceArray(32 * 4096)
 with A.HipAttentionLibrary(0) as hip:
-    call(hip, [A.WEIGHTS_Q8_0], 32, 4096, small, out)
+    call(hip, [Q8_0], 32, 4096)
     before = live()
-    call(hip, [A.WEIGHTS_Q4_K, A.WEIGHTS_Q6_K], 16, 8192, small, out)
-    call(hip, [A.WEIGHTS_Q6_K], 17, 7680, small, out)
+    captured(hip, [Q4_K, Q6_K], 16, 8192)
+    captured(hip, [Q6_K], 17, 7680)
     assert live() == before, "a call of no more activations grew the scratch"
 """)
 
